@@ -27,6 +27,15 @@
 
 namespace trixi_hip {
 
+// A coefficient: on the device kept in scalar registers (the compiler
+// otherwise copies each one into vector registers, two moves per step).
+TRIXI_FASTLOG_QUAL double fastlog_const(double c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+s"(c));
+#endif
+    return c;
+}
+
 TRIXI_FASTLOG_QUAL double fast_log(double x) {
     int e;
     double m = std::frexp(x, &e);  // x = m 2^e, m in [1/2, 1) for positive finite x
@@ -40,15 +49,15 @@ TRIXI_FASTLOG_QUAL double fast_log(double x) {
     const double z = s * s;
     // 1 + z/3 + z^2/5 + ... + z^9/19 (Horner, explicit fused multiply-adds so
     // that host and device round alike)
-    double q = 1.0 / 19.0;
-    q = std::fma(q, z, 1.0 / 17.0);
-    q = std::fma(q, z, 1.0 / 15.0);
-    q = std::fma(q, z, 1.0 / 13.0);
-    q = std::fma(q, z, 1.0 / 11.0);
-    q = std::fma(q, z, 1.0 / 9.0);
-    q = std::fma(q, z, 1.0 / 7.0);
-    q = std::fma(q, z, 1.0 / 5.0);
-    q = std::fma(q, z, 1.0 / 3.0);
+    double q = fastlog_const(1.0 / 19.0);
+    q = std::fma(q, z, fastlog_const(1.0 / 17.0));
+    q = std::fma(q, z, fastlog_const(1.0 / 15.0));
+    q = std::fma(q, z, fastlog_const(1.0 / 13.0));
+    q = std::fma(q, z, fastlog_const(1.0 / 11.0));
+    q = std::fma(q, z, fastlog_const(1.0 / 9.0));
+    q = std::fma(q, z, fastlog_const(1.0 / 7.0));
+    q = std::fma(q, z, fastlog_const(1.0 / 5.0));
+    q = std::fma(q, z, fastlog_const(1.0 / 3.0));
     // log(m) = 2 s + 2 s z q
     const double two_s = 2.0 * s;
     const double logm = std::fma(two_s, z * q, two_s);

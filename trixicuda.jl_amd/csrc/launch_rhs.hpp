@@ -1,0 +1,73 @@
+// launch_rhs.hpp -- which form of the rhs! kernel a configuration runs.
+#pragma once
+
+#include "rhs_group_kernel.hpp"
+
+namespace trixi_hip {
+
+// Shapes of the lane-group form: FP64 flux differencing and shock capturing in
+// 2D and 3D for the equations with a rotation, whole waves per group.
+template <class EQ>
+struct HasRotation : std::false_type {};
+template <int DIM>
+struct HasRotation<Euler<DIM>> : std::true_type {};
+template <>
+struct HasRotation<GlmMhd> : std::true_type {};
+
+#ifndef TRIXI_HIP_GROUP_LDS_KIB
+#define TRIXI_HIP_GROUP_LDS_KIB 78
+#endif
+// Elements per workgroup: the most (a power of two) whose LDS leaves room for
+// two workgroups per compute unit, at most 16.
+template <int DIM, int N, int NV, int NRF>
+constexpr int group_elems() {
+    constexpr int NL = cpow(N, DIM - 1), NN = cpow(N, DIM);
+    int m = 16;
+    while (m > 1 && m * 8 * (NRF * NN + NV * NN + DIM * 2 * NL * NV) > TRIXI_HIP_GROUP_LDS_KIB * 1024) m /= 2;
+    return m;
+}
+#ifndef TRIXI_HIP_GROUP_WAVES2D
+#define TRIXI_HIP_GROUP_WAVES2D 3
+#endif
+template <int DIM, int N, class EQ, int VOL, typename R>
+constexpr bool group_eligible() {
+    return std::is_same<R, double>::value && DIM > 1 && VOL != VI_WEAK && HasRotation<EQ>::value &&
+           (group_elems<DIM, N, EQ::NV, EQ::NRF>() * cpow(N, DIM - 1)) % 64 == 0 &&
+           group_threads<DIM, N, group_elems<DIM, N, EQ::NV, EQ::NRF>()>() <= 1024;
+}
+
+// Launch helper used by the instantiation units: the node-parallel form for
+// small periodic conforming meshes (RhsArgs::np), the lane-group form where it
+// is built, the line form otherwise.
+template <int DIM, int N, class EQ, int VOL, int VF, int SF, int FVF, typename R, int M, bool RK, bool EXT = false,
+          typename L = double, typename S = double>
+hipError_t launch_rhs(const RhsArgs& a, hipStream_t stream) {
+    auto grid = [&](int m) {
+        int64_t blocks = (a.E + m - 1) / m;
+        if (a.nxcd > 1) blocks = (blocks + a.nxcd - 1) / a.nxcd * a.nxcd;
+        return dim3((unsigned)blocks);
+    };
+    if constexpr (np_eligible<DIM, N, EQ::NV, VOL, EXT>()) {
+        if (a.np) {
+            constexpr int MN = np_elems<DIM, N>();
+            hipLaunchKernelGGL((rhs_np_kernel<DIM, N, EQ, VOL, VF, SF, FVF, R, RK, L, S>), grid(MN),
+                               dim3(MN * cpow(N, DIM) * DIM), 0, stream, a);
+            return hipGetLastError();
+        }
+    }
+    // only the node-parallel form computes the next stage's blending factors
+    if (a.alpha_next != nullptr) return hipErrorInvalidValue;
+    if constexpr (group_eligible<DIM, N, EQ, VOL, R>()) {
+        constexpr int ME = group_elems<DIM, N, EQ::NV, EQ::NRF>();
+        constexpr int MG = EXT && (ME / 2 * cpow(N, DIM - 1)) % 64 == 0 ? ME / 2 : ME;
+        constexpr int W = EQ::NV > 5 || EXT ? 2 : (DIM == 3 ? 4 : TRIXI_HIP_GROUP_WAVES2D);
+        hipLaunchKernelGGL((rhs_group_kernel<DIM, N, EQ, VOL, VF, SF, FVF, MG, RK, EXT, W>), grid(MG),
+                           dim3(group_threads<DIM, N, MG>()), 0, stream, a);
+    } else {
+        hipLaunchKernelGGL((rhs_kernel<DIM, N, EQ, VOL, VF, SF, FVF, R, M, RK, EXT, L, S>), grid(M),
+                           dim3(rhs_threads<DIM, N, M, R, RK, EQ::NV>()), 0, stream, a);
+    }
+    return hipGetLastError();
+}
+
+}  // namespace trixi_hip

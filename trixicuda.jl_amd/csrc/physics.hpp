@@ -108,17 +108,19 @@ __device__ __forceinline__ int64_t soa(int v, int node, int64_t e, int64_t slab,
 
 // ---------------------------------------------------------------------------
 // arithmetic helpers.
-//   FP64: reciprocal = v_rcp_f64 refined by two Newton steps, quotient
-//         n * r corrected by one residual step (within about 1 ulp, far
-//         inside the FP64 parity bound, 6 instructions instead of the
-//         11-instruction IEEE sequence); IEEE square root.
+//   FP64: reciprocal = v_rcp_f64 (relative error below 2^-24, measured)
+//         refined by one third-order step r (1 + e + e^2), e = 1 - d r (the
+//         remaining e^3 is below 2^-72), quotient n * r corrected by one
+//         residual step (within about 1 ulp, far inside the FP64 parity
+//         bound, 6 instructions instead of the 11-instruction IEEE sequence);
+//         square root = v_rsq_f64 with one coupled (Goldschmidt) step and one
+//         residual correction (within 1 ulp; 0 and infinity as they are).
 //   FP32 (mixed mode): v_rcp_f32 and v_sqrt_f32 (within 2 ulp of FP32).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ double rrcp(double d) {
-    double r = __builtin_amdgcn_rcp(d);
-    r = fma(fma(-d, r, 1.0), r, r);
-    r = fma(fma(-d, r, 1.0), r, r);
-    return r;
+    const double r = __builtin_amdgcn_rcp(d);
+    const double e = fma(-d, r, 1.0);
+    return fma(r, fma(e, e, e), r);
 }
 __device__ __forceinline__ float rrcp(float d) { return __builtin_amdgcn_rcpf(d); }
 __device__ __forceinline__ double rdiv(double n, double d) {
@@ -127,7 +129,15 @@ __device__ __forceinline__ double rdiv(double n, double d) {
     return fma(fma(-d, q, n), r, q);
 }
 __device__ __forceinline__ float rdiv(float n, float d) { return n * __builtin_amdgcn_rcpf(d); }
-__device__ __forceinline__ double rsqrt_(double x) { return sqrt(x); }
+__device__ __forceinline__ double rsqrt_(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double e = fma(-h, g, 0.5);
+    g = fma(g, e, g);
+    h = fma(h, e, h);
+    g = fma(fma(-g, g, x), h, g);
+    return __builtin_amdgcn_class(x, 0x260) ? x : g;  // 0x260: -0, +0, +inf
+}
 __device__ __forceinline__ float rsqrt_(float x) { return __builtin_amdgcn_sqrtf(x); }
 __device__ __forceinline__ double dabs(double x) { return fabs(x); }
 __device__ __forceinline__ float dabs(float x) { return fabsf(x); }
@@ -177,6 +187,74 @@ __device__ __forceinline__ R inv_ln_mean_logs(R x, R y, L lx, L ly) {
     const R z = dxy * r, f2 = z * z;
     const R pp = R(2) + f2 * (R(2.0 / 3.0) + f2 * (R(2.0 / 5.0) + f2 * R(2.0 / 7.0)));
     return series ? pp * r : dl * r;
+}
+
+// ---------------------------------------------------------------------------
+// The two logarithmic means of an entropy-conservative flux without node
+// logarithms (FP64 arithmetic): ln_mean(x1, y1) and inv_ln_mean(x2, y2) with
+// one reciprocal for both, from the series in z^2, z = (y - x) / (x + y).
+//   log(y / x) = z P(z^2), P(q) = 2 atanh(sqrt q) / sqrt q, and Q = 1 / P:
+//   minimax polynomials of degree 6 for |z| < 0.15 (y / x < 1.353), relative
+//   error below 3e-17 (P) and 6e-18 (Q), so the result is the mean's to
+//   round-off.
+// MEANS_NEAR: the caller knows that |z| < 0.15 for both.  MEANS_ANY: any
+// x, y; lanes further apart take the closed form with the logarithm of the
+// quotient, in a block that a wave without such lanes skips.
+// Against node logarithms (two per node, staged in LDS) with a three-term
+// series below |z| = 0.01, the FP64 kernels drop the logarithms, their LDS and
+// registers, and every select and branch of a pair.
+// ---------------------------------------------------------------------------
+constexpr int MEANS_NEAR = 1, MEANS_ANY = 2;
+
+// v_min_f64 / v_max_f64 as they are (fmin and fmax first quiet each operand
+// with an instruction of its own); a NaN operand yields the other one
+__device__ __forceinline__ double raw_min(double x, double y) {
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+    return r;
+}
+__device__ __forceinline__ double raw_max(double x, double y) {
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+    return r;
+}
+// y / x < 1.15 / 0.85 for x <= y (false for x <= 0 and for NaN)
+__device__ __forceinline__ bool near_ratio(double x, double y) { return 0.85 * y < 1.15 * x; }
+
+template <int MEANS>
+__device__ __forceinline__ void log_free_means(double x1, double y1, double x2, double y2, double& mean1,
+                                               double& inv_mean2) {
+    const double s1 = x1 + y1, d1 = y1 - x1;
+    const double s2 = x2 + y2, d2 = y2 - x2;
+    const double r = rrcp(s1 * s2);
+    const double r1 = r * s2, r2 = r * s1;
+    const double z1 = d1 * r1, z2 = d2 * r2;
+    const double q1 = z1 * z1, q2 = z2 * z2;
+    double Q = fma(q1, fastlog_const(-0.008948152998574805), fastlog_const(-0.01088099532782093));
+    Q = fma(q1, Q, fastlog_const(-0.015097271029888403));
+    Q = fma(q1, Q, fastlog_const(-0.023280421147242054));
+    Q = fma(q1, Q, fastlog_const(-0.0444444444524844));
+    Q = fma(q1, Q, fastlog_const(-0.1666666666666553));
+    Q = fma(q1, Q, 0.5);
+    double Pq = fma(q2, fastlog_const(0.16481117002486795), fastlog_const(0.1814740093132822));
+    Pq = fma(q2, Pq, fastlog_const(0.2222275413776025));
+    Pq = fma(q2, Pq, fastlog_const(0.28571424363123693));
+    Pq = fma(q2, Pq, fastlog_const(0.4000000001583343));
+    Pq = fma(q2, Pq, fastlog_const(0.6666666666664435));
+    Pq = fma(q2, Pq, 2.0);
+    mean1 = s1 * Q;
+    inv_mean2 = Pq * r2;
+    if constexpr (MEANS == MEANS_ANY) {
+        // (false for nonpositive sums and NaN, which then go through the logarithm)
+        const bool near1 = fabs(d1) < 0.15 * s1, near2 = fabs(d2) < 0.15 * s2;
+        if (__builtin_amdgcn_ballot_w64(!(near1 && near2)) != 0) {
+            const double nan = __builtin_nan("");
+            const double l1 = x1 > 0.0 ? fast_log(rdiv(y1, x1)) : nan;
+            const double l2 = x2 > 0.0 ? fast_log(rdiv(y2, x2)) : nan;
+            mean1 = near1 ? mean1 : rdiv(d1, l1);
+            inv_mean2 = near2 ? inv_mean2 : rdiv(l2, d2);
+        }
+    }
 }
 
 // ===========================================================================
@@ -431,6 +509,96 @@ struct Euler {
         f[DIM + 1] = (n.cons(DIM + 1) + n.p) * n.v[o];
     }
 
+    // flux_ranocha from its logarithmic means
+    template <typename R, typename L>
+    __device__ static void ranocha(const Node<R, L>& l, const Node<R, L>& r, int o, const PhysR<R>& P, R rho_mean,
+                                   R inv_rho_p_mean, R* f) {
+        R vavg[DIM];
+        R vsq = R(0);
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+            vavg[d] = R(0.5) * (l.v[d] + r.v[d]);
+            vsq = (d == 0) ? l.v[d] * r.v[d] : vsq + l.v[d] * r.v[d];
+        }
+        const R velocity_square_avg = R(0.5) * vsq;
+        const R p_avg = R(0.5) * (l.p + r.p);
+        const R f1 = rho_mean * vavg[o];
+        f[0] = f1;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) f[1 + d] = (d == o) ? f1 * vavg[d] + p_avg : f1 * vavg[d];
+        f[DIM + 1] = f1 * (velocity_square_avg + inv_rho_p_mean * P.inv_gm1) +
+                     R(0.5) * (l.p * r.v[o] + r.p * l.v[o]);
+    }
+
+    // Twice a two-point flux (FP64): the factors 1/2 of the averages and of the
+    // Lax-Friedrichs flux go into the kernel's final factor.
+    // FLUX_RANOCHA without node logarithms: with V = v_l + v_r and h = ln_mean(rho) V_o / 2,
+    //   2 f = (2 h, h V + (p_l + p_r) e_o,
+    //          h (v_l . v_r + 2 / (gamma - 1) p_l p_r inv_ln_mean) + p_l v_r,o + p_r v_l,o).
+    // FLUX_SHIMA_ETAL: the same with h = (rho_l + rho_r) V_o / 4 and the
+    // energy's internal part (p_l + p_r) V_o / (2 (gamma - 1)).
+    // FLUX_LLF*: with the conservative states u_l, u_r,
+    //   2 f = v_l,o u_l + v_r,o u_r + lambda (u_l - u_r) + (0, (p_l + p_r) e_o, p_l v_l,o + p_r v_r,o).
+    template <int KIND, int MEANS, typename L>
+    __device__ static void twice_flux(const Node<double, L>& l, const double* ul, const Node<double, L>& r,
+                                      const double* ur, int o, const PhysR<double>& P, double* f) {
+        if constexpr (KIND == FLUX_SHIMA_ETAL) {
+            const double Vo = l.v[o] + r.v[o], psum = l.p + r.p;
+            f[0] = 0.5 * ((l.rho + r.rho) * Vo);
+            const double h = 0.5 * f[0];
+            double vsq = l.v[0] * r.v[0];
+#pragma unroll
+            for (int d = 1; d < DIM; ++d) vsq = fma(l.v[d], r.v[d], vsq);
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) f[1 + d] = (d == o) ? fma(h, Vo, psum) : h * (l.v[d] + r.v[d]);
+            const double e = fma(l.p, r.v[o], r.p * l.v[o]);
+            f[DIM + 1] = fma(h, vsq, fma(0.5 * P.inv_gm1, psum * Vo, e));
+        } else if constexpr (KIND == FLUX_RANOCHA) {
+            double rho_mean, inv_mean;
+            log_free_means<MEANS>(l.rho, r.rho, l.rho * r.p, r.rho * l.p, rho_mean, inv_mean);
+            const double Vo = l.v[o] + r.v[o];
+            f[0] = rho_mean * Vo;
+            const double h = 0.5 * f[0];
+            double vsq = l.v[0] * r.v[0];
+#pragma unroll
+            for (int d = 1; d < DIM; ++d) vsq = fma(l.v[d], r.v[d], vsq);
+#pragma unroll
+            for (int d = 0; d < DIM; ++d)
+                f[1 + d] = (d == o) ? fma(h, Vo, l.p + r.p) : h * (l.v[d] + r.v[d]);
+            const double e = fma(l.p, r.v[o], r.p * l.v[o]);
+            f[DIM + 1] = fma(h, fma(l.p * r.p * inv_mean, 2.0 * P.inv_gm1, vsq), e);
+        } else {
+            double lam;
+            if (KIND == FLUX_LLF_NAIVE)
+                lam = dmax(dabs(l.v[o]), dabs(r.v[o])) + dmax(l.c, r.c);
+            else
+                lam = dmax(dabs(l.v[o]) + l.c, dabs(r.v[o]) + r.c);
+#pragma unroll
+            for (int q = 0; q < NV; ++q) {
+                double t = fma(l.v[o], ul[q], r.v[o] * ur[q]);
+                if (q == 1 + o) t += l.p + r.p;
+                if (q == DIM + 1) t = fma(l.p, l.v[o], fma(r.p, r.v[o], t));
+                f[q] = fma(lam, ul[q] - ur[q], t);
+            }
+        }
+    }
+    // whether every pair of these nodes satisfies MEANS_NEAR: rho, and rho / p
+    // through the staged sound speed (rho / p = gamma / c^2)
+    template <int N, typename L>
+    __device__ static bool near_line(const Node<double, L>* n) {
+        double r0 = n[0].rho, r1 = r0, c0 = n[0].c, c1 = c0, p0 = n[0].p;
+#pragma unroll
+        for (int i = 1; i < N; ++i) {
+            r0 = raw_min(r0, n[i].rho);
+            r1 = raw_max(r1, n[i].rho);
+            c0 = raw_min(c0, n[i].c);
+            c1 = raw_max(c1, n[i].c);
+            p0 = raw_min(p0, n[i].p);
+        }
+        const bool a = near_ratio(r0, r1), b = near_ratio(c0 * c0, c1 * c1), c = p0 > 0.0;
+        return a && b && c;
+    }
+
     template <int KIND, typename R, typename L>
     __device__ static void two_point(const Node<R, L>& l, const Node<R, L>& r, int o, const PhysR<R>& P, R* f) {
         if (KIND == FLUX_RANOCHA) {
@@ -438,21 +606,7 @@ struct Euler {
             // p_ll p_rr inv_ln_mean(rho_ll p_rr, rho_rr p_ll), logs log(rho)+log(p)
             const R inv_rho_p_mean =
                 l.p * r.p * inv_ln_mean_logs<R>(l.rho * r.p, r.rho * l.p, l.lrho + r.lp, r.lrho + l.lp);
-            R vavg[DIM];
-            R vsq = R(0);
-#pragma unroll
-            for (int d = 0; d < DIM; ++d) {
-                vavg[d] = R(0.5) * (l.v[d] + r.v[d]);
-                vsq = (d == 0) ? l.v[d] * r.v[d] : vsq + l.v[d] * r.v[d];
-            }
-            const R velocity_square_avg = R(0.5) * vsq;
-            const R p_avg = R(0.5) * (l.p + r.p);
-            const R f1 = rho_mean * vavg[o];
-            f[0] = f1;
-#pragma unroll
-            for (int d = 0; d < DIM; ++d) f[1 + d] = (d == o) ? f1 * vavg[d] + p_avg : f1 * vavg[d];
-            f[DIM + 1] = f1 * (velocity_square_avg + inv_rho_p_mean * P.inv_gm1) +
-                         R(0.5) * (l.p * r.v[o] + r.p * l.v[o]);
+            ranocha(l, r, o, P, rho_mean, inv_rho_p_mean, f);
         } else if (KIND == FLUX_SHIMA_ETAL) {
             const R rho_avg = R(0.5) * (l.rho + r.rho);
             R vavg[DIM];
@@ -1115,44 +1269,77 @@ struct GlmMhd {
         cf = rsqrt_(R(0.5) * (a2 + b2 + astar));
     }
 
+    // flux_hindenlang_gassner from its logarithmic means
+    template <typename R, typename L>
+    __device__ static void hindenlang_gassner(const Node<R, L>& l, const Node<R, L>& r, int o, const PhysR<R>& P,
+                                              R rho_mean, R inv_rho_p_mean, R* f) {
+        const R* Bl = l.B;
+        const R* Br = r.B;
+        const R psil = l.psi, psir = r.psi;
+        R vavg[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) vavg[d] = R(0.5) * (l.v[d] + r.v[d]);
+        const R p_avg = R(0.5) * (l.p + r.p);
+        const R psi_avg = R(0.5) * (psil + psir);
+        const R velocity_square_avg = R(0.5) * (l.v[0] * r.v[0] + l.v[1] * r.v[1] + l.v[2] * r.v[2]);
+        const R magnetic_square_avg = R(0.5) * (Bl[0] * Br[0] + Bl[1] * Br[1] + Bl[2] * Br[2]);
+        const R f1 = rho_mean * vavg[o];
+        f[0] = f1;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            R t = f1 * vavg[d];
+            if (d == o) t = t + p_avg + magnetic_square_avg;
+            f[1 + d] = t - R(0.5) * (Bl[o] * Br[d] + Br[o] * Bl[d]);
+        }
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+            f[5 + d] = (d == o) ? P.c_h * psi_avg
+                                : R(0.5) * (l.v[o] * Bl[d] - l.v[d] * Bl[o] + r.v[o] * Br[d] - r.v[d] * Br[o]);
+        f[8] = P.c_h * R(0.5) * (Bl[o] + Br[o]);
+        R s = l.p * r.v[o] + r.p * l.v[o];
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+            if (d != o) s = s + (l.v[o] * Bl[d] * Br[d] + r.v[o] * Br[d] * Bl[d]);
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+            if (d != o) s = s - (l.v[d] * Bl[o] * Br[d] + r.v[d] * Br[o] * Bl[d]);
+        s = s + P.c_h * (Bl[o] * psir + Br[o] * psil);
+        f[4] = f1 * (velocity_square_avg + inv_rho_p_mean * P.inv_gm1) + R(0.5) * s;
+    }
+
+    // flux_hindenlang_gassner without node logarithms (FP64)
+    template <int KIND, int MEANS, typename L>
+    __device__ static void two_point_log_free(const Node<double, L>& l, const Node<double, L>& r, int o,
+                                              const PhysR<double>& P, double* f) {
+        static_assert(KIND == FLUX_HINDENLANG_GASSNER, "the flux with logarithmic means");
+        double rho_mean, inv_mean;
+        log_free_means<MEANS>(l.rho, r.rho, l.rho * r.p, r.rho * l.p, rho_mean, inv_mean);
+        hindenlang_gassner(l, r, o, P, rho_mean, l.p * r.p * inv_mean, f);
+    }
+    // whether every pair of these nodes satisfies MEANS_NEAR: rho, and rho / p
+    // (v_rcp_f64 as it is: within 2^-24, far inside the polynomials' margin)
+    template <int N, typename L>
+    __device__ static bool near_line(const Node<double, L>* n) {
+        double r0 = n[0].rho, r1 = r0, b0 = r0 * __builtin_amdgcn_rcp(n[0].p), b1 = b0;
+#pragma unroll
+        for (int i = 1; i < N; ++i) {
+            const double b = n[i].rho * __builtin_amdgcn_rcp(n[i].p);
+            r0 = raw_min(r0, n[i].rho);
+            r1 = raw_max(r1, n[i].rho);
+            b0 = raw_min(b0, b);
+            b1 = raw_max(b1, b);
+        }
+        const bool a = near_ratio(r0, r1), b = near_ratio(b0, b1);
+        return a && b;
+    }
+
     template <int KIND, typename R, typename L>
     __device__ static void two_point(const Node<R, L>& l, const Node<R, L>& r, int o, const PhysR<R>& P, R* f) {
         if (KIND == FLUX_HINDENLANG_GASSNER) {
-            const R* Bl = l.B;
-            const R* Br = r.B;
-            const R psil = l.psi, psir = r.psi;
             const R rho_mean = ln_mean_logs<R>(l.rho, r.rho, l.lrho, r.lrho);
             const R inv_rho_p_mean =
                 l.p * r.p * inv_ln_mean_logs<R>(l.rho * r.p, r.rho * l.p, l.lrho + r.lp, r.lrho + l.lp);
-            R vavg[3];
-#pragma unroll
-            for (int d = 0; d < 3; ++d) vavg[d] = R(0.5) * (l.v[d] + r.v[d]);
-            const R p_avg = R(0.5) * (l.p + r.p);
-            const R psi_avg = R(0.5) * (psil + psir);
-            const R velocity_square_avg = R(0.5) * (l.v[0] * r.v[0] + l.v[1] * r.v[1] + l.v[2] * r.v[2]);
-            const R magnetic_square_avg = R(0.5) * (Bl[0] * Br[0] + Bl[1] * Br[1] + Bl[2] * Br[2]);
-            const R f1 = rho_mean * vavg[o];
-            f[0] = f1;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                R t = f1 * vavg[d];
-                if (d == o) t = t + p_avg + magnetic_square_avg;
-                f[1 + d] = t - R(0.5) * (Bl[o] * Br[d] + Br[o] * Bl[d]);
-            }
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-                f[5 + d] = (d == o) ? P.c_h * psi_avg
-                                    : R(0.5) * (l.v[o] * Bl[d] - l.v[d] * Bl[o] + r.v[o] * Br[d] - r.v[d] * Br[o]);
-            f[8] = P.c_h * R(0.5) * (Bl[o] + Br[o]);
-            R s = l.p * r.v[o] + r.p * l.v[o];
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-                if (d != o) s = s + (l.v[o] * Bl[d] * Br[d] + r.v[o] * Br[d] * Bl[d]);
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-                if (d != o) s = s - (l.v[d] * Bl[o] * Br[d] + r.v[d] * Br[o] * Bl[d]);
-            s = s + P.c_h * (Bl[o] * psir + Br[o] * psil);
-            f[4] = f1 * (velocity_square_avg + inv_rho_p_mean * P.inv_gm1) + R(0.5) * s;
+            hindenlang_gassner(l, r, o, P, rho_mean, inv_rho_p_mean, f);
         } else {
             R fl[9], fr[9];
             flux(l, o, P, fl);
@@ -1290,5 +1477,43 @@ struct GlmMhd1D {
         GlmMhd::max_abs_speeds(u9, P, lam);
     }
 };
+
+// FP64 kernels of compressible Euler whose fluxes all have a doubled form
+// (twice_flux): they accumulate twice every term and halve once at the end.
+template <class EQ>
+struct IsEuler : std::false_type {};
+template <int DIM>
+struct IsEuler<Euler<DIM>> : std::true_type {};
+constexpr bool twice_kind(int k) {
+    return k == FLUX_RANOCHA || k == FLUX_SHIMA_ETAL || k == FLUX_LLF || k == FLUX_LLF_NAIVE;
+}
+template <class EQ, typename R, int VOL, int VF, int SF, int FVF>
+constexpr bool twice_fluxes() {
+    return IsEuler<EQ>::value && std::is_same<R, double>::value && VOL != VI_WEAK && twice_kind(VF) &&
+           twice_kind(SF) && (VOL != VI_HG || twice_kind(FVF));
+}
+// FP64 kernels that take the logarithmic means without node logarithms
+// (every Euler kernel with such a flux has the doubled form).
+template <class EQ, typename R, bool TWICE>
+constexpr bool log_free() {
+    return TWICE || (std::is_same<EQ, GlmMhd>::value && std::is_same<R, double>::value);
+}
+
+// Two-point flux: twice the flux where TWICE (ul, ur: the conservative states
+// of the nodes, read by the Lax-Friedrichs kinds only), otherwise from nodes
+// that carry logarithms where their flux and arithmetic type need them.
+template <class EQ, int KIND, bool TWICE, int MEANS, typename R, typename L>
+__device__ __forceinline__ void node_flux(const typename EQ::template Node<R, L>& l, const R* ul,
+                                          const typename EQ::template Node<R, L>& r, const R* ur, int o,
+                                          const PhysR<R>& P, R* f) {
+    if constexpr (TWICE)
+        EQ::template twice_flux<KIND, MEANS>(l, ul, r, ur, o, P, f);
+    else if constexpr (log_free<EQ, R, TWICE>() && flux_needs_logs(KIND))
+        EQ::template two_point_log_free<KIND, MEANS>(l, r, o, P, f);
+    else
+        EQ::template two_point<KIND>(l, r, o, P, f);
+}
+// whether a node_flux of this kind reads the conservative states
+constexpr bool flux_reads_cons(bool twice, int k) { return twice && (k == FLUX_LLF || k == FLUX_LLF_NAIVE); }
 
 }  // namespace trixi_hip

@@ -1,8 +1,8 @@
 // registry.hpp -- table of the compiled rhs kernel instantiations.
 #pragma once
 
+#include "launch_rhs.hpp"
 #include "mortar_kernel.hpp"
-#include "rhs_kernel.hpp"
 #include "vjp_kernel.hpp"
 
 namespace trixi_hip {

@@ -266,7 +266,11 @@ rhs_kernel(const RhsArgs a) {
     constexpr bool SF_LOGS = flux_needs_logs(SF);
     constexpr bool VF_LOGS = (VOL != VI_WEAK) && flux_needs_logs(VF);
     constexpr bool FV_LOGS = (VOL == VI_HG) && flux_needs_logs(FVF);
-    constexpr bool NODE_LOGS = SF_LOGS || VF_LOGS || FV_LOGS;
+    // FP64 Euler: fluxes and accumulators hold twice their value (TW); no node
+    // logarithms there, nor in the FP64 MHD kernels (LF)
+    constexpr bool TW = twice_fluxes<EQ, R, VOL, VF, SF, FVF>();
+    constexpr bool LF = log_free<EQ, R, TW>();
+    constexpr bool NODE_LOGS = !LF && (SF_LOGS || VF_LOGS || FV_LOGS);
     constexpr int NDF = NODE_LOGS ? 2 : 0;
     using Node = typename EQ::template Node<R, L>;
     // mixed precision weak form with N = 4 on whole waves: D-hat on MFMA
@@ -456,7 +460,7 @@ rhs_kernel(const RhsArgs a) {
 
     // last direction, sequential or not: -1/J (+ sources), then du or the RK update
     auto line_epilogue = [&](R (&al)[N][NV], int base, int s) {
-        const double fac = -a.invJ[e];
+        const double fac = (TW ? -0.5 : -1.0) * a.invJ[e];
         double t_dt = 0.0;
         if (RK) t_dt = a.time[1];
 #pragma unroll
@@ -480,6 +484,39 @@ rhs_kernel(const RhsArgs a) {
                     UO[g] = (S)((double)U[g] + a.rk_b * (double)kk);
                 }
             }
+        }
+    };
+
+    auto staged_node = [&](int node) {
+        R f[NRF];
+#pragma unroll
+        for (int k = 0; k < NRF; ++k) f[k] = rec[(k * NN + node) * LDM + el];
+        const L lr = NODE_LOGS ? recd[node * LDM + el] : L(0);
+        const L lp = NODE_LOGS ? recd[(NN + node) * LDM + el] : L(0);
+        return EQ::from_rec(f, lr, lp, P);
+    };
+
+    // the pairs of a line whose nodes lie too far apart for the series means:
+    // one pair per turn, its nodes from LDS, added to all nodes with weight
+    // zero for the others (registers are not indexed dynamically)
+    auto line_pairs_any = [&](int d, int base, int s, R sc, R (&al)[N][NV]) {
+        if constexpr (LF && VF_LOGS) {
+#pragma unroll 1
+            for (int i = 0; i + 1 < N; ++i)
+#pragma unroll 1
+                for (int j = i + 1; j < N; ++j) {
+                    R f[NV];
+                    node_flux<EQ, VF, TW, MEANS_ANY, R, L>(staged_node(base + i * s), nullptr,
+                                                           staged_node(base + j * s), nullptr, d, P, f);
+                    const R fa = sc * (R)a.Ds[i * N + j];
+                    const R fb = sc * (R)a.Ds[j * N + i];
+#pragma unroll
+                    for (int p = 0; p < N; ++p) {
+                        const R w = p == i ? fa : (p == j ? fb : R(0));
+#pragma unroll
+                        for (int v = 0; v < NV; ++v) al[p][v] += w * f[v];
+                    }
+                }
         }
     };
 
@@ -540,12 +577,7 @@ rhs_kernel(const RhsArgs a) {
         for (int p = 0; p < N; ++p) {
             const int node = base + p * s;
             if (STAGE) {
-                R f[NRF];
-#pragma unroll
-                for (int k = 0; k < NRF; ++k) f[k] = rec[(k * NN + node) * LDM + el];
-                const L lr = NODE_LOGS ? recd[node * LDM + el] : L(0);
-                const L lp = NODE_LOGS ? recd[(NN + node) * LDM + el] : L(0);
-                nd[p] = EQ::from_rec(f, lr, lp, P);
+                nd[p] = staged_node(node);
             } else {
                 R uc[NV];
 #pragma unroll
@@ -595,20 +627,35 @@ rhs_kernel(const RhsArgs a) {
             }
         } else {
             const R sc = (VOL == VI_HG && !dg_only) ? R(1) - alpha : R(1);
+            // one decision per wave and line where the flux takes logarithmic
+            // means without node logarithms (LF): every pair close enough for
+            // the series (branch free, all pairs in flight together), or else
+            // one pair at a time with its checks (a jump of more than a third)
+            bool near = true;
+            if constexpr (LF && VF_LOGS)
+                near = __builtin_amdgcn_ballot_w64(!EQ::template near_line<N>(nd)) == 0;
+            if (near) {
 #pragma unroll
-            for (int i = 0; i < N; ++i)
+                for (int i = 0; i < N; ++i)
 #pragma unroll
-                for (int j = i + 1; j < N; ++j) {
-                    R f[NV];
-                    EQ::template two_point<VF>(nd[i], nd[j], d, P, f);
-                    const R fa = sc * (R)a.Ds[i * N + j];
-                    const R fb = sc * (R)a.Ds[j * N + i];
+                    for (int j = i + 1; j < N; ++j) {
+                        R f[NV];
+                        node_flux<EQ, VF, TW, MEANS_NEAR, R, L>(nd[i], nullptr, nd[j], nullptr, d, P, f);
+                        const R fa = sc * (R)a.Ds[i * N + j];
+                        const R fb = sc * (R)a.Ds[j * N + i];
 #pragma unroll
-                    for (int v = 0; v < NV; ++v) {
-                        acl[i][v] += fa * f[v];
-                        acl[j][v] += fb * f[v];
+                        for (int v = 0; v < NV; ++v) {
+                            acl[i][v] += fa * f[v];
+                            acl[j][v] += fb * f[v];
+                        }
                     }
-                }
+            } else if constexpr (LF && VF_LOGS) {
+                line_pairs_any(d, base, s, sc, acl);
+                // (read again, so that they hold no registers above)
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int p = 0; p < N; ++p) nd[p] = staged_node(base + p * s);
+            }
             if constexpr (EQ::NONCONS) {
 #pragma unroll
                 for (int i = 0; i < N; ++i) {
@@ -631,8 +678,15 @@ rhs_kernel(const RhsArgs a) {
             if (VOL == VI_HG && !dg_only) {
 #pragma unroll
                 for (int p = 0; p + 1 < N; ++p) {
-                    R F[NV];
-                    EQ::template two_point<FVF>(nd[p], nd[p + 1], d, P, F);
+                    R F[NV], ul[NV], ur[NV];
+                    if constexpr (flux_reads_cons(TW, FVF)) {
+#pragma unroll
+                        for (int v = 0; v < NV; ++v) {
+                            ul[v] = nd[p].cons(v);
+                            ur[v] = nd[p + 1].cons(v);
+                        }
+                    }
+                    node_flux<EQ, FVF, TW, MEANS_ANY, R, L>(nd[p], ul, nd[p + 1], ur, d, P, F);
                     const R wl = alpha * (R)a.invw[p];
                     const R wr = alpha * (R)a.invw[p + 1];
                     if constexpr (EQ::NONCONS) {
@@ -659,11 +713,19 @@ rhs_kernel(const RhsArgs a) {
 
         // ---- interface fluxes at both ends of the line, surface integral ----
         {
-            const Node ndm = EQ::template node<R, SF_LOGS, L>(um, P);
-            const Node ndp = EQ::template node<R, SF_LOGS, L>(up, P);
+            const Node ndm = EQ::template node<R, SF_LOGS && NODE_LOGS, L>(um, P);
+            const Node ndp = EQ::template node<R, SF_LOGS && NODE_LOGS, L>(up, P);
             R fm[NV], fp[NV];
-            EQ::template two_point<SF>(ndm, nd[0], d, P, fm);       // this element is "right"
-            EQ::template two_point<SF>(nd[N - 1], ndp, d, P, fp);   // this element is "left"
+            R u0[NV], u1[NV];
+            if constexpr (flux_reads_cons(TW, SF)) {
+#pragma unroll
+                for (int v = 0; v < NV; ++v) {
+                    u0[v] = nd[0].cons(v);
+                    u1[v] = nd[N - 1].cons(v);
+                }
+            }
+            node_flux<EQ, SF, TW, MEANS_ANY, R, L>(ndm, um, nd[0], u0, d, P, fm);      // this element is "right"
+            node_flux<EQ, SF, TW, MEANS_ANY, R, L>(nd[N - 1], u1, ndp, up, d, P, fp);  // this element is "left"
             if constexpr (EQ::NONCONS) {
                 R ncm[NV], ncp[NV];
                 EQ::template noncons<SF>(nd[0], ndm, d, P, ncm);
@@ -679,12 +741,12 @@ rhs_kernel(const RhsArgs a) {
                 if (nb[2 * d] <= -2) {
                     const double* mf = a.mflux + ((int64_t)(-2 - nb[2 * d]) * NL + line) * NV;
 #pragma unroll
-                    for (int v = 0; v < NV; ++v) fm[v] = (R)mf[v];
+                    for (int v = 0; v < NV; ++v) fm[v] = (TW ? R(2) : R(1)) * (R)mf[v];
                 }
                 if (nb[2 * d + 1] <= -2) {
                     const double* mf = a.mflux + ((int64_t)(-2 - nb[2 * d + 1]) * NL + line) * NV;
 #pragma unroll
-                    for (int v = 0; v < NV; ++v) fp[v] = (R)mf[v];
+                    for (int v = 0; v < NV; ++v) fp[v] = (TW ? R(2) : R(1)) * (R)mf[v];
                 }
             }
             const R lm = (R)a.lhat_m, lp = (R)a.lhat_p;
@@ -761,7 +823,7 @@ rhs_kernel(const RhsArgs a) {
             const int n = q / M;
             const int64_t ee = e0 + c;
             if (ee >= E) continue;
-            const double fac = -a.invJ[ee];
+            const double fac = (TW ? -0.5 : -1.0) * a.invJ[ee];
             double sv[NV];
 #pragma unroll
             for (int v = 0; v < NV; ++v) sv[v] = 0.0;
@@ -837,7 +899,10 @@ rhs_np_kernel(const RhsArgs a) {
     constexpr bool SF_LOGS = flux_needs_logs(SF);
     constexpr bool VF_LOGS = flux_needs_logs(VF);
     constexpr bool FV_LOGS = (VOL == VI_HG) && flux_needs_logs(FVF);
-    constexpr bool NODE_LOGS = SF_LOGS || VF_LOGS || FV_LOGS;
+    // FP64 Euler: fluxes and accumulators hold twice their value (TW); no node
+    // logarithms there, nor in the FP64 MHD kernels (LF)
+    constexpr bool TW = twice_fluxes<EQ, R, VOL, VF, SF, FVF>();
+    constexpr bool NODE_LOGS = !log_free<EQ, R, TW>() && (SF_LOGS || VF_LOGS || FV_LOGS);
     constexpr int NDF = NODE_LOGS ? 2 : 0;
     using Node = typename EQ::template Node<R, L>;
     static_assert(VOL != VI_WEAK, "the node-parallel form is built for flux differencing and HG");
@@ -919,6 +984,9 @@ rhs_np_kernel(const RhsArgs a) {
         return EQ::from_rec(f, lr, lq, P);
     };
     const Node me = load_node(node);
+    R ume[NV];  // its conservative state, where a flux reads it
+#pragma unroll
+    for (int v = 0; v < NV; ++v) ume[v] = TW ? me.cons(v) : R(0);
 
     R acl[NV];
 #pragma unroll
@@ -956,7 +1024,7 @@ rhs_np_kernel(const RhsArgs a) {
             const Node lo = select_node<EQ, R, L>(below, other, me, P);
             const Node hi = select_node<EQ, R, L>(below, me, other, P);
             R f[NV];
-            EQ::template two_point<VF>(lo, hi, D, P, f);
+            node_flux<EQ, VF, TW, MEANS_ANY, R, L>(lo, nullptr, hi, nullptr, D, P, f);
             const R w = sc * (below ? dsr[q] : dsr[q + 1]);
     #pragma unroll
             for (int v = 0; v < NV; ++v) acl[v] += w * f[v];
@@ -982,8 +1050,12 @@ rhs_np_kernel(const RhsArgs a) {
             const R w = alpha * invw_p;
             if (p > 0) {  // subcell interface p - 1/2: this node is its right node
                 const Node left = load_node(node - SD);
-                R F[NV];
-                EQ::template two_point<FVF>(left, me, D, P, F);
+                R F[NV], un[NV];
+                if constexpr (flux_reads_cons(TW, FVF)) {
+    #pragma unroll
+                    for (int v = 0; v < NV; ++v) un[v] = left.cons(v);
+                }
+                node_flux<EQ, FVF, TW, MEANS_ANY, R, L>(left, un, me, ume, D, P, F);
                 if constexpr (EQ::NONCONS) {
                     R nc[NV];
                     EQ::template noncons<FVF>(me, left, D, P, nc);
@@ -996,8 +1068,12 @@ rhs_np_kernel(const RhsArgs a) {
             }
             if (p < N - 1) {  // subcell interface p + 1/2: this node is its left node
                 const Node right = load_node(node + SD);
-                R F[NV];
-                EQ::template two_point<FVF>(me, right, D, P, F);
+                R F[NV], un[NV];
+                if constexpr (flux_reads_cons(TW, FVF)) {
+    #pragma unroll
+                    for (int v = 0; v < NV; ++v) un[v] = right.cons(v);
+                }
+                node_flux<EQ, FVF, TW, MEANS_ANY, R, L>(me, ume, right, un, D, P, F);
                 if constexpr (EQ::NONCONS) {
                     R nc[NV];
                     EQ::template noncons<FVF>(me, right, D, P, nc);
@@ -1013,12 +1089,19 @@ rhs_np_kernel(const RhsArgs a) {
         // interface flux at the line's ends and its surface-integral weight
         // (this element is "right" at its -d face, "left" at its +d face)
         if (face) {
-            const Node nb = EQ::template node<R, SF_LOGS, L>(ub, P);
+            const Node nb = EQ::template node<R, SF_LOGS && NODE_LOGS, L>(ub, P);
             const bool minus = p == 0;
             const Node lo = select_node<EQ, R, L>(minus, nb, me, P);
             const Node hi = select_node<EQ, R, L>(minus, me, nb, P);
-            R fs[NV];
-            EQ::template two_point<SF>(lo, hi, D, P, fs);
+            R fs[NV], ulo[NV], uhi[NV];
+            if constexpr (flux_reads_cons(TW, SF)) {
+    #pragma unroll
+                for (int v = 0; v < NV; ++v) {
+                    ulo[v] = minus ? ub[v] : ume[v];
+                    uhi[v] = minus ? ume[v] : ub[v];
+                }
+            }
+            node_flux<EQ, SF, TW, MEANS_ANY, R, L>(lo, ulo, hi, uhi, D, P, fs);
             if constexpr (EQ::NONCONS) {
                 R nc[NV];
                 EQ::template noncons<SF>(me, nb, D, P, nc);
@@ -1048,7 +1131,7 @@ rhs_np_kernel(const RhsArgs a) {
     // (no early exit: the fused indicator below synchronises the workgroup)
     double uo[FUSE_IND ? NV : 1];
     if (last && valid) {
-        const double fac = -a.invJ[e];
+        const double fac = (TW ? -0.5 : -1.0) * a.invJ[e];
         double t_dt = 0.0;
         if (RK) t_dt = a.time[1];
 #pragma unroll
@@ -1117,30 +1200,6 @@ rhs_np_kernel(const RhsArgs a) {
 template <int DIM, int N, int NV, int VOL, bool EXT>
 __host__ __device__ constexpr bool np_eligible() {
     return !EXT && VOL != VI_WEAK && DIM > 1 && NV <= 5 && cpow(N, DIM) * DIM <= 1024;
-}
-
-// Launch helper used by the instantiation units: the node-parallel form for
-// small periodic conforming meshes (RhsArgs::np), the line form otherwise.
-template <int DIM, int N, class EQ, int VOL, int VF, int SF, int FVF, typename R, int M, bool RK, bool EXT = false,
-          typename L = double, typename S = double>
-hipError_t launch_rhs(const RhsArgs& a, hipStream_t stream) {
-    if constexpr (np_eligible<DIM, N, EQ::NV, VOL, EXT>()) {
-        if (a.np) {
-            constexpr int MN = np_elems<DIM, N>();
-            int64_t blocks = (a.E + MN - 1) / MN;
-            if (a.nxcd > 1) blocks = (blocks + a.nxcd - 1) / a.nxcd * a.nxcd;
-            hipLaunchKernelGGL((rhs_np_kernel<DIM, N, EQ, VOL, VF, SF, FVF, R, RK, L, S>), dim3((unsigned)blocks),
-                               dim3(MN * cpow(N, DIM) * DIM), 0, stream, a);
-            return hipGetLastError();
-        }
-    }
-    // only the node-parallel form computes the next stage's blending factors
-    if (a.alpha_next != nullptr) return hipErrorInvalidValue;
-    int64_t blocks = (a.E + M - 1) / M;
-    if (a.nxcd > 1) blocks = (blocks + a.nxcd - 1) / a.nxcd * a.nxcd;
-    hipLaunchKernelGGL((rhs_kernel<DIM, N, EQ, VOL, VF, SF, FVF, R, M, RK, EXT, L, S>), dim3((unsigned)blocks),
-                       dim3(rhs_threads<DIM, N, M, R, RK, EQ::NV>()), 0, stream, a);
-    return hipGetLastError();
 }
 
 }  // namespace trixi_hip
