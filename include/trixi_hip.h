@@ -328,6 +328,11 @@ int trixi_hip_rk_step_f32(trixi_hip_ctx* ctx, float* u, float* k, double t, doub
 int trixi_hip_max_dt(trixi_hip_ctx* ctx, const double* u, double* max_dt,
                      trixi_hip_stream stream);
 
+/* trixi_hip_max_dt of an FP32 state (contexts of precision TRIXI_HIP_FP32; each
+ * value widened, so the result is that of the widened state). */
+int trixi_hip_max_dt_f32(trixi_hip_ctx* ctx, const float* u, double* max_dt,
+                         trixi_hip_stream stream);
+
 /* trixi_hip_max_dt without any allocation: the block partials and the maximum
  * go to a static device scratch of 2048 doubles (16 KiB, held by every GPU
  * the library runs on until the process ends) instead of the context's

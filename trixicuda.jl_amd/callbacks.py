@@ -14,9 +14,10 @@ from .semidiscretization import _ptr, _stream
 
 
 def max_dt(u_ode, semi):
-    u_ode = semi.as_f64(u_ode, "u_ode")
+    semi.check_vector(u_ode, "u_ode")
     out = ctypes.c_double()
-    L.check(L.lib().trixi_hip_max_dt(semi.ctx, _ptr(u_ode), ctypes.byref(out), _stream()))
+    fn = L.lib().trixi_hip_max_dt_f32 if semi.fp32_state else L.lib().trixi_hip_max_dt
+    L.check(fn(semi.ctx, _ptr(u_ode), ctypes.byref(out), _stream()))
     return out.value
 
 

@@ -16,6 +16,7 @@
 #include "registry.hpp"
 #include "initial_conditions.hpp"
 #include "indicator.hpp"
+#include "reductions.hpp"
 
 namespace trixi_hip {
 
@@ -604,162 +605,10 @@ __global__ void set_time_kernel(double* time, double t, double dt, double c0, do
     }
 }
 
-// Per-element max_abs_speeds scaled by invJ, reduced per block (max).
-template <class EQ, int DIM>
-__global__ void max_speed_kernel(const double* __restrict__ u, const double* __restrict__ invJ,
-                                 double* __restrict__ partial, int nn, int64_t E, PhysParams phys) {
-    __shared__ double red[256];
-    const PhysR<double> P = PhysR<double>::from(phys);
-    double best = 0.0;
-    for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < E;
-         e += (int64_t)gridDim.x * blockDim.x) {
-        double lmax[3] = {0, 0, 0};
-        for (int n = 0; n < nn; ++n) {
-            double uc[EQ::NV], lam[3];
-            for (int v = 0; v < EQ::NV; ++v) uc[v] = u[((int64_t)v * nn + n) * E + e];
-            EQ::max_abs_speeds(uc, P, lam);
-            for (int d = 0; d < DIM; ++d) lmax[d] = lam[d] > lmax[d] ? lam[d] : lmax[d];
-        }
-        double s = 0.0;
-        for (int d = 0; d < DIM; ++d) s += lmax[d];
-        const double sc = invJ[e] * s;
-        best = sc > best ? sc : best;
-    }
-    red[threadIdx.x] = best;
-    __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + w]);
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
-}
-
-// Deterministic final reduction of `nblocks` partial vectors of length m:
-// components [0, nsum) are summed, [nsum, m) take the maximum; one thread
-// per component, fixed order.
-__global__ void reduce_partials_kernel(const double* __restrict__ partial, double* __restrict__ out,
-                                       int nblocks, int m, int nsum) {
-    const int c = threadIdx.x;
-    if (c >= m) return;
-    const bool is_sum = c < nsum;
-    double acc = is_sum ? 0.0 : partial[c];
-    for (int b = is_sum ? 0 : 1; b < nblocks; ++b) {
-        const double v = partial[(int64_t)b * m + c];
-        acc = is_sum ? acc + v : fmax(acc, v);
-    }
-    out[c] = acc;
-}
-
-// Error norms: each thread handles analysis points (element, analysis node),
-// interpolating u and x with the (NA x N) Vandermonde of the 2N analysis
-// basis.  Block partials: [l2 (nv) | linf (nv)].
-template <int DIM>
-__global__ void error_norms_kernel(const double* __restrict__ u, const double* __restrict__ xs,
-                                   const double* __restrict__ invJ, double* __restrict__ partial,
-                                   const double* __restrict__ Vdm_g, const double* __restrict__ wa_g,
-                                   int N, int NA, int64_t E, IcParams q, double t, int nv) {
-    __shared__ double red[256 * 18];
-    const int nn = (int)lrint(pow((double)N, (double)DIM));
-    const int nna = (int)lrint(pow((double)NA, (double)DIM));
-    double l2[9], li[9];
-    for (int v = 0; v < nv; ++v) {
-        l2[v] = 0.0;
-        li[v] = 0.0;
-    }
-    const int64_t total = (int64_t)nna * E;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t e = i / nna;
-        const int a = (int)(i % nna);
-        int ai[3] = {0, 0, 0};
-        {
-            int r = a;
-            for (int d = 0; d < DIM; ++d) {
-                ai[d] = r % NA;
-                r /= NA;
-            }
-        }
-        double ua[9], xa[3] = {0, 0, 0};
-        for (int v = 0; v < nv; ++v) ua[v] = 0.0;
-        for (int n = 0; n < nn; ++n) {
-            double w = 1.0;
-            int r = n;
-            for (int d = 0; d < DIM; ++d) {
-                w *= Vdm_g[ai[d] * N + (r % N)];
-                r /= N;
-            }
-            if (w == 0.0) continue;
-            for (int v = 0; v < nv; ++v) ua[v] += w * u[((int64_t)v * nn + n) * E + e];
-            for (int d = 0; d < DIM; ++d) xa[d] += w * xs[((int64_t)d * nn + n) * E + e];
-        }
-        double uex[9];
-        initial_condition(q, xa, t, 0, uex);
-        double wq = 1.0;
-        for (int d = 0; d < DIM; ++d) wq *= wa_g[ai[d]];
-        const double vj = pow(1.0 / invJ[e], (double)DIM);
-        for (int v = 0; v < nv; ++v) {
-            const double diff = uex[v] - ua[v];
-            l2[v] += diff * diff * (wq * vj);
-            li[v] = fmax(li[v], fabs(diff));
-        }
-    }
-    for (int v = 0; v < nv; ++v) {
-        red[threadIdx.x * 18 + v] = l2[v];
-        red[threadIdx.x * 18 + 9 + v] = li[v];
-    }
-    __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w)
-            for (int v = 0; v < nv; ++v) {
-                red[threadIdx.x * 18 + v] += red[(threadIdx.x + w) * 18 + v];
-                red[threadIdx.x * 18 + 9 + v] =
-                    fmax(red[threadIdx.x * 18 + 9 + v], red[(threadIdx.x + w) * 18 + 9 + v]);
-            }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0)
-        for (int v = 0; v < nv; ++v) {
-            partial[(int64_t)blockIdx.x * 2 * nv + v] = red[v];
-            partial[(int64_t)blockIdx.x * 2 * nv + nv + v] = red[9 + v];
-        }
-}
-
-__global__ void integrate_kernel(const double* __restrict__ u, const double* __restrict__ invJ,
-                                 double* __restrict__ partial, const double* __restrict__ w_g, int N,
-                                 int dim, int64_t E, int nv) {
-    __shared__ double red[256 * 9];
-    int nn = 1;
-    for (int d = 0; d < dim; ++d) nn *= N;
-    double acc[9];
-    for (int v = 0; v < nv; ++v) acc[v] = 0.0;
-    for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < E;
-         e += (int64_t)gridDim.x * blockDim.x) {
-        const double vj = pow(1.0 / invJ[e], (double)dim);
-        for (int n = 0; n < nn; ++n) {
-            double w = 1.0;
-            int r = n;
-            for (int d = 0; d < dim; ++d) {
-                w *= w_g[r % N];
-                r /= N;
-            }
-            for (int v = 0; v < nv; ++v) acc[v] += vj * w * u[((int64_t)v * nn + n) * E + e];
-        }
-    }
-    for (int v = 0; v < nv; ++v) red[threadIdx.x * 9 + v] = acc[v];
-    __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w)
-            for (int v = 0; v < nv; ++v) red[threadIdx.x * 9 + v] += red[(threadIdx.x + w) * 9 + v];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0)
-        for (int v = 0; v < nv; ++v) partial[(int64_t)blockIdx.x * nv + v] = red[v];
-}
-
 // Positivity / finiteness flags per element (FP64).
 __global__ void check_state_kernel(const double* __restrict__ u, int32_t* __restrict__ flags,
-                                   double* __restrict__ partial, int eq, int dim, int nv, int nn,
-                                   int64_t E, PhysParams phys) {
+                                   double* __restrict__ partial, double* out, unsigned* arrived, int eq, int dim,
+                                   int nv, int nn, int64_t E, PhysParams phys) {
     __shared__ double red[256];
     double cnt = 0.0;
     for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < E;
@@ -815,7 +664,8 @@ __global__ void check_state_kernel(const double* __restrict__ u, int32_t* __rest
         if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
         __syncthreads();
     }
-    if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
+    if (threadIdx.x == 0) store_partial(&partial[blockIdx.x], red[0]);
+    finish_partials<256>(partial, out, arrived, 1, 1);
 }
 
 }  // namespace trixi_hip
@@ -841,7 +691,8 @@ struct trixi_hip_ctx {
     double* d_alpha = nullptr;
     double* d_time = nullptr;
     double* d_partial = nullptr;
-    double* d_result = nullptr;
+    double* h_result = nullptr;    // pinned: the last block of a reduction writes here
+    unsigned* d_arrived = nullptr;  // blocks of a running reduction that have arrived
     double* d_Vinv = nullptr;
     double* d_Vdm = nullptr;
     double* d_wa = nullptr;
@@ -922,11 +773,12 @@ static void free_ctx(trixi_hip_ctx* c) {
     if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
     if (c->graph) (void)hipGraphDestroy(c->graph);
     void* bufs[] = {c->d_nbr, c->d_invJ, c->d_x,     c->d_alpha_raw, c->d_alpha, c->d_time,
-                    c->d_partial, c->d_result, c->d_Vinv, c->d_Vdm,   c->d_wa,    c->d_w,
+                    c->d_partial, c->d_arrived, c->d_Vinv, c->d_Vdm,   c->d_wa,    c->d_w,
                     c->d_tmp, c->d_stage, c->d_k, c->d_kbar, c->d_alphabar, c->d_winner, c->d_stage_alpha,
                     c->d_mids, c->d_mori, c->d_mls, c->d_mnb, c->d_mflux};
     for (void* p : bufs)
         if (p) (void)hipFree(p);
+    if (c->h_result) (void)hipHostFree(c->h_result);
     delete c;
 }
 
@@ -1273,7 +1125,11 @@ int trixi_hip_create(const trixi_hip_config* config, const trixi_hip_mesh* mesh,
     ALLOC(c->d_alpha, E * sizeof(double));
     ALLOC(c->d_time, 16 * sizeof(double));
     ALLOC(c->d_partial, (size_t)c->nblocks_red * 18 * sizeof(double));
-    ALLOC(c->d_result, 32 * sizeof(double));
+    ALLOC(c->d_arrived, sizeof(unsigned));
+    if (hipHostMalloc((void**)&c->h_result, 32 * sizeof(double), hipHostMallocMapped) != hipSuccess)
+        return cleanup_fail(TRIXI_HIP_ENOMEM, "hipHostMalloc failed for the reduction results");
+    if (hipMemset(c->d_arrived, 0, sizeof(unsigned)) != hipSuccess)
+        return cleanup_fail(TRIXI_HIP_EDEVICE, "hipMemset failed in create");
     ALLOC(c->d_Vinv, N * N * sizeof(double));
     ALLOC(c->d_Vdm, c->NA * N * sizeof(double));
     ALLOC(c->d_wa, c->NA * sizeof(double));
@@ -1664,15 +1520,22 @@ static int rk_step_any(trixi_hip_ctx* ctx, void* u, void* k, double t, double dt
     return TRIXI_HIP_OK;
 }
 
-// max_dt with its block partials in `partial` (at least `blocks` doubles) and
-// the reduced maximum in `result`.
-static int max_dt_impl(trixi_hip_ctx* ctx, const double* u, double* max_dt, hipStream_t s, int blocks,
-                       double* partial, double* result) {
-    const int threads = 256;
+// Blocks of an element reduction (at most nblocks_red, four per compute unit).
+static int reduction_blocks(const trixi_hip_ctx* c) {
+    return (int)std::min<int64_t>((c->E + RED_ELEMS - 1) / RED_ELEMS, c->nblocks_red);
+}
+
+// The largest scaled wave speed of u (of type S) into `result`, which the
+// device writes, with the block partials in `partial` (at least `blocks`
+// doubles) and the arrival count in `arrived` (zero before and after).
+extern "C++" template <typename S>
+static int launch_max_speed(trixi_hip_ctx* ctx, const S* u, hipStream_t s, int blocks, double* partial,
+                            double* result, unsigned* arrived) {
     const PhysParams& P = ctx->args.phys;
     const int eq = ctx->cfg.equation, dim = ctx->dim;
-#define MS(EQT, D) \
-    hipLaunchKernelGGL((max_speed_kernel<EQT, D>), dim3(blocks), dim3(threads), 0, s, u, ctx->d_invJ, partial, ctx->nn, ctx->E, P)
+#define MS(EQT, D)                                                                                                 \
+    hipLaunchKernelGGL((max_speed_kernel<EQT, D, S>), dim3(blocks), dim3(RED_THREADS), 0, s, u, ctx->d_invJ, partial, \
+                       result, arrived, ctx->nn, ctx->E, P)
     if (eq == TRIXI_HIP_LINEAR_SCALAR_ADVECTION) {
         if (dim == 1) MS(LinAdv<1>, 1); else if (dim == 2) MS(LinAdv<2>, 2); else MS(LinAdv<3>, 3);
     } else if (eq == TRIXI_HIP_COMPRESSIBLE_EULER) {
@@ -1701,37 +1564,71 @@ static int max_dt_impl(trixi_hip_ctx* ctx, const double* u, double* max_dt, hipS
     }
 #undef MS
     HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(32), 0, s, partial, result, blocks, 1, 0);
-    HIP_TRY(hipGetLastError());
-    double m = 0.0;
-    HIP_TRY(hipMemcpyAsync(&m, result, sizeof(double), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    return TRIXI_HIP_OK;
+}
+
+static double max_dt_of(const trixi_hip_ctx* ctx, double m) {
     const double tiny = nextafter(0.0, 1.0);
     if (!(m > tiny)) m = tiny;
-    *max_dt = 2.0 / (ctx->N * m);
+    return 2.0 / (ctx->N * m);
+}
+
+extern "C++" template <typename S>
+static int max_dt_any(trixi_hip_ctx* ctx, const S* u, double* max_dt, hipStream_t s) {
+    int rc = launch_max_speed(ctx, u, s, reduction_blocks(ctx), ctx->d_partial, ctx->h_result, ctx->d_arrived);
+    if (rc) return rc;
+    HIP_TRY(hipStreamSynchronize(s));
+    *max_dt = max_dt_of(ctx, ctx->h_result[0]);
     return TRIXI_HIP_OK;
 }
 
 int trixi_hip_max_dt(trixi_hip_ctx* ctx, const double* u, double* max_dt, trixi_hip_stream stream) {
     if (!ctx || !u || !max_dt) return fail(TRIXI_HIP_EINVAL, "null argument");
-    const int blocks = (int)std::min<int64_t>((ctx->E + 255) / 256, ctx->nblocks_red);
-    return max_dt_impl(ctx, u, max_dt, (hipStream_t)stream, blocks, ctx->d_partial, ctx->d_result);
+    return max_dt_any(ctx, u, max_dt, (hipStream_t)stream);
+}
+
+int trixi_hip_max_dt_f32(trixi_hip_ctx* ctx, const float* u, double* max_dt, trixi_hip_stream stream) {
+    if (!ctx || !u || !max_dt) return fail(TRIXI_HIP_EINVAL, "null argument");
+    if (!fp32_state(ctx)) return fail(TRIXI_HIP_EINVAL, "this context's state is FP64: use trixi_hip_max_dt");
+    return max_dt_any(ctx, u, max_dt, (hipStream_t)stream);
 }
 
 int trixi_hip_max_dt_noalloc(trixi_hip_ctx* ctx, const double* u, double* max_dt, trixi_hip_stream stream) {
     if (!ctx || !u || !max_dt) return fail(TRIXI_HIP_EINVAL, "null argument");
     // the same grid as trixi_hip_max_dt: the same partials and maximum
-    const int blocks = (int)std::min<int64_t>((ctx->E + 255) / 256, ctx->nblocks_red);
-    if (blocks + 1 > TRIXI_HIP_SCRATCH_DOUBLES)
+    const int blocks = reduction_blocks(ctx);
+    if (blocks + 2 > TRIXI_HIP_SCRATCH_DOUBLES)
         return fail(TRIXI_HIP_EINVAL, "max_dt_noalloc: " + std::to_string(blocks) +
                                           " block partials exceed the static scratch of " +
-                                          std::to_string(TRIXI_HIP_SCRATCH_DOUBLES - 1));
+                                          std::to_string(TRIXI_HIP_SCRATCH_DOUBLES - 2));
     double* sp = nullptr;
-    const int rc = scratch_ptr(&sp);
+    int rc = scratch_ptr(&sp);
     if (rc) return rc;
-    // partials in [0, blocks), the maximum in the last slot; every partial is
-    // written before it is read, so nothing needs clearing between calls
-    return max_dt_impl(ctx, u, max_dt, (hipStream_t)stream, blocks, sp, sp + TRIXI_HIP_SCRATCH_DOUBLES - 1);
+    // partials in [0, blocks), the arrival count and the maximum in the last
+    // two slots; every partial is written before it is read, and the count is
+    // zero at load and left at zero, so nothing needs clearing between calls
+    hipStream_t s = (hipStream_t)stream;
+    double* const result = sp + TRIXI_HIP_SCRATCH_DOUBLES - 1;
+    rc = launch_max_speed(ctx, u, s, blocks, sp, result,
+                          reinterpret_cast<unsigned*>(sp + TRIXI_HIP_SCRATCH_DOUBLES - 2));
+    if (rc) return rc;
+    double m = 0.0;
+    HIP_TRY(hipMemcpyAsync(&m, result, sizeof(double), hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    *max_dt = max_dt_of(ctx, m);
+    return TRIXI_HIP_OK;
+}
+
+extern "C++" template <int DIM, int N>
+static hipError_t launch_error_norms(trixi_hip_ctx* ctx, const double* u, const IcParams& q, double t, hipStream_t s) {
+    // a wave per element, as many waves as 60 KiB of LDS take
+    const size_t wave_bytes = en_wave_doubles<DIM, N>(ctx->nv) * sizeof(double);
+    const int waves = wave_bytes * 4 <= 60 * 1024 ? 4 : (wave_bytes * 2 <= 60 * 1024 ? 2 : 1);
+    const int blocks = (int)std::min<int64_t>((ctx->E + waves - 1) / waves, ctx->nblocks_red);
+    hipLaunchKernelGGL((error_norms_kernel<DIM, N>), dim3(blocks), dim3(64 * waves), (unsigned)(waves * wave_bytes), s,
+                       u, ctx->d_x, ctx->d_invJ, ctx->d_partial, ctx->h_result, ctx->d_arrived, ctx->d_Vdm, ctx->d_wa,
+                       ctx->E, q, t, ctx->nv);
+    return hipGetLastError();
 }
 
 int trixi_hip_error_norms(trixi_hip_ctx* ctx, const double* u, int32_t ic, double t, uint64_t seed, double* l2,
@@ -1739,26 +1636,29 @@ int trixi_hip_error_norms(trixi_hip_ctx* ctx, const double* u, int32_t ic, doubl
     if (!ctx || !u || !l2 || !linf) return fail(TRIXI_HIP_EINVAL, "null argument");
     if (ic < 0 || ic > TRIXI_HIP_IC_HARMONIC_NONPERIODIC) return fail(TRIXI_HIP_EINVAL, "unknown initial condition");
     hipStream_t s = (hipStream_t)stream;
-    const int threads = 256;
-    const int64_t npts = (int64_t)ctx->E * (int64_t)lrint(pow((double)ctx->NA, (double)ctx->dim));
-    const int blocks = (int)std::min<int64_t>((npts + threads - 1) / threads, ctx->nblocks_red);
     const IcParams q = ic_params(ctx, ic, seed);
     const int nv = ctx->nv;
-#define EN(D)                                                                                                   \
-    hipLaunchKernelGGL((error_norms_kernel<D>), dim3(blocks), dim3(threads), 0, s, u, ctx->d_x, ctx->d_invJ,    \
-                       ctx->d_partial, ctx->d_Vdm, ctx->d_wa, ctx->N, ctx->NA, ctx->E, q, t, nv)
-    if (ctx->dim == 1) EN(1); else if (ctx->dim == 2) EN(2); else EN(3);
+    hipError_t e = hipErrorInvalidValue;
+#define EN(NQ)                                                       \
+    case NQ:                                                         \
+        e = ctx->dim == 1   ? launch_error_norms<1, NQ>(ctx, u, q, t, s) \
+            : ctx->dim == 2 ? launch_error_norms<2, NQ>(ctx, u, q, t, s) \
+                            : launch_error_norms<3, NQ>(ctx, u, q, t, s); \
+        break
+    switch (ctx->N) {
+        EN(2);
+        EN(3);
+        EN(4);
+        EN(5);
+        default:
+            return fail(TRIXI_HIP_EUNSUPPORTED, "error norms are built for polydeg 1 to 4");
+    }
 #undef EN
-    HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(32), 0, s, ctx->d_partial, ctx->d_result, blocks,
-                       2 * nv, nv);
-    HIP_TRY(hipGetLastError());
-    double res[18];
-    HIP_TRY(hipMemcpyAsync(res, ctx->d_result, 2 * nv * sizeof(double), hipMemcpyDeviceToHost, s));
+    HIP_TRY(e);
     HIP_TRY(hipStreamSynchronize(s));
     for (int v = 0; v < nv; ++v) {
-        l2[v] = sqrt(res[v] / ctx->total_volume);
-        linf[v] = res[nv + v];
+        l2[v] = sqrt(ctx->h_result[v] / ctx->total_volume);
+        linf[v] = ctx->h_result[nv + v];
     }
     return TRIXI_HIP_OK;
 }
@@ -1766,16 +1666,14 @@ int trixi_hip_error_norms(trixi_hip_ctx* ctx, const double* u, int32_t ic, doubl
 int trixi_hip_integrate(trixi_hip_ctx* ctx, const double* u, double* integral, trixi_hip_stream stream) {
     if (!ctx || !u || !integral) return fail(TRIXI_HIP_EINVAL, "null argument");
     hipStream_t s = (hipStream_t)stream;
-    const int threads = 256;
-    const int blocks = (int)std::min<int64_t>((ctx->E + threads - 1) / threads, ctx->nblocks_red);
-    hipLaunchKernelGGL(integrate_kernel, dim3(blocks), dim3(threads), 0, s, u, ctx->d_invJ, ctx->d_partial,
-                       ctx->d_w, ctx->N, ctx->dim, ctx->E, ctx->nv);
+#define IK(D)                                                                                                        \
+    hipLaunchKernelGGL((integrate_kernel<D>), dim3(reduction_blocks(ctx)), dim3(RED_THREADS), 0, s, u, ctx->d_invJ,    \
+                       ctx->d_partial, ctx->h_result, ctx->d_arrived, ctx->d_w, ctx->N, ctx->nn, ctx->E, ctx->nv)
+    if (ctx->dim == 1) IK(1); else if (ctx->dim == 2) IK(2); else IK(3);
+#undef IK
     HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(32), 0, s, ctx->d_partial, ctx->d_result, blocks,
-                       ctx->nv, ctx->nv);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(integral, ctx->d_result, ctx->nv * sizeof(double), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
+    for (int v = 0; v < ctx->nv; ++v) integral[v] = ctx->h_result[v];
     return TRIXI_HIP_OK;
 }
 
@@ -2031,14 +1929,10 @@ int trixi_hip_check_state(trixi_hip_ctx* ctx, const double* u, int32_t* flags, i
     const int threads = 256;
     const int blocks = (int)std::min<int64_t>((ctx->E + threads - 1) / threads, ctx->nblocks_red);
     hipLaunchKernelGGL(check_state_kernel, dim3(blocks), dim3(threads), 0, s, u, flags, ctx->d_partial,
-                       ctx->cfg.equation, ctx->dim, ctx->nv, ctx->nn, ctx->E, ctx->args.phys);
+                       ctx->h_result, ctx->d_arrived, ctx->cfg.equation, ctx->dim, ctx->nv, ctx->nn, ctx->E, ctx->args.phys);
     HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(32), 0, s, ctx->d_partial, ctx->d_result, blocks, 1, 1);
-    HIP_TRY(hipGetLastError());
-    double cnt = 0.0;
-    HIP_TRY(hipMemcpyAsync(&cnt, ctx->d_result, sizeof(double), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
-    *nbad = (int64_t)cnt;
+    *nbad = (int64_t)ctx->h_result[0];
     if (*nbad > 0) return fail(TRIXI_HIP_ESTATE, std::to_string(*nbad) + " element(s) with invalid state");
     return TRIXI_HIP_OK;
 }
