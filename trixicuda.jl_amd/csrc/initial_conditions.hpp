@@ -180,6 +180,15 @@ __device__ inline void weak_blast_prim(const IcParams& q, const double* x, uint6
     }
 }
 
+// The travelling waves of initial_condition_convergence_test: compressible
+// Euler's density (xs: sum of the coordinates) and linear advection's solution
+// (xs: sum of x_d - a_d t).
+__device__ __forceinline__ double euler_wave(double xs, double t) { return 2.0 + 0.1 * sin(M_PI * (xs - t)); }
+__device__ __forceinline__ double advection_wave(double xs) {
+    const double omega = 2.0 * M_PI * (1.0 / 2.0);
+    return 1.0 + 0.5 * sin(omega * xs);
+}
+
 // Initial conditions (Trixi initial_condition_* functions used by the
 // reference tests and examples, plus the seeded benchmark states).
 __device__ inline void initial_condition(const IcParams& q, const double* x, double t, uint64_t idx,
@@ -270,8 +279,7 @@ __device__ inline void initial_condition(const IcParams& q, const double* x, dou
         if (q.ic == TRIXI_HIP_IC_CONVERGENCE_TEST) {
             double xs = 0.0;
             for (int d = 0; d < q.dim; ++d) xs += x[d] - q.a[d] * t;
-            const double omega = 2.0 * M_PI * (1.0 / 2.0);
-            u[0] = 1.0 + 0.5 * sin(omega * xs);
+            u[0] = advection_wave(xs);
         } else if (q.ic == TRIXI_HIP_IC_SEEDED_RANDOM) {
             u[0] = 1.0 + 0.1 * (2.0 * u01(q.seed, idx, 0) - 1.0);
         } else {
@@ -303,7 +311,7 @@ __device__ inline void initial_condition(const IcParams& q, const double* x, dou
         } else if (q.ic == TRIXI_HIP_IC_CONVERGENCE_TEST) {
             double xs = 0.0;
             for (int d = 0; d < q.dim; ++d) xs += x[d];
-            const double ini = 2.0 + 0.1 * sin(M_PI * (xs - t));
+            const double ini = euler_wave(xs, t);
             u[0] = ini;
             for (int d = 0; d < q.dim; ++d) u[1 + d] = ini;
             u[q.dim + 1] = ini * ini;

@@ -44,9 +44,19 @@ __device__ __forceinline__ void finish_partials(const double* partial, double* o
     for (int c = wave; c < m; c += THREADS / 64) {
         const bool sum = c < nsum;
         double x = 0.0;  // the maxima are of values >= 0
-        for (int b = lane; b < (int)gridDim.x; b += 64) {
-            const double y = __hip_atomic_load(&partial[(int64_t)b * m + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            x = sum ? x + y : fmax(x, y);
+        // eight loads in flight (each goes past the caches: one at a time they
+        // were most of a call)
+        for (int b0 = lane; b0 < (int)gridDim.x; b0 += 64 * 8) {
+            double y[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int b = b0 + 64 * i;
+                y[i] = b < (int)gridDim.x ? __hip_atomic_load(&partial[(int64_t)b * m + c], __ATOMIC_RELAXED,
+                                                              __HIP_MEMORY_SCOPE_AGENT)
+                                          : 0.0;
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x = sum ? x + y[i] : fmax(x, y[i]);
         }
 #pragma unroll
         for (int w = 32; w > 0; w >>= 1) {
@@ -135,12 +145,13 @@ __device__ __forceinline__ void block_sums(double x, double* red, double* dst) {
 }
 
 // sum_e J_e^d sum_n w_n u: each group of 16 lanes its nodes of 16 elements.
-template <int DIM>
+template <int DIM, int N>
 __global__ void __launch_bounds__(RED_THREADS) integrate_kernel(const double* __restrict__ u,
                                                                 const double* __restrict__ invJ,
                                                                 double* __restrict__ partial, double* out,
                                                                 unsigned* arrived, const double* __restrict__ w_g,
-                                                                int N, int nn, int64_t E, int nv) {
+                                                                int64_t E, int nv) {
+    constexpr int nn = cpow(N, DIM);
     __shared__ double red[RED_THREADS / 64];
     const int c = threadIdx.x % RED_ELEMS, g = threadIdx.x / RED_ELEMS;
     double acc[9];
@@ -153,6 +164,7 @@ __global__ void __launch_bounds__(RED_THREADS) integrate_kernel(const double* __
         double vj = h;
 #pragma unroll
         for (int d = 1; d < DIM; ++d) vj *= h;
+#pragma unroll 4
         for (int n = g; n < nn; n += RED_GROUPS) {
             double w = vj;
             int r = n;
@@ -183,13 +195,19 @@ constexpr int en_wave_doubles(int nv) {
     constexpr int NA = 2 * N - 1;
     return nv * (DIM > 1 ? NA * cpow(N, DIM - 1) : 0) + nv * (DIM > 2 ? NA * NA * N : 0) + DIM * NA;
 }
-template <int DIM, int N>
+// EXACT: the state compared against.  The waves of the convergence tests, which
+// error norms are mostly taken against, have kernels of their own; the others
+// go through the general function, a call per point with its registers and stack
+// (82 us against 48 at 4096 elements of 3D Euler).
+constexpr int EN_GENERAL = 0, EN_EULER_WAVE = 1, EN_ADVECTION_WAVE = 2;
+template <int DIM, int N, int EXACT>
 __global__ void __launch_bounds__(256) error_norms_kernel(const double* __restrict__ u, const double* __restrict__ xs,
                                                           const double* __restrict__ invJ,
                                                           double* __restrict__ partial, double* out,
                                                           unsigned* arrived, const double* __restrict__ Vdm_g,
-                                                          const double* __restrict__ wa_g, int64_t E, IcParams q0,
-                                                          double t, int nv) {
+                                                          const double* __restrict__ wa_g, int64_t E, IcParams q,
+                                                          double t, int nv_) {
+    const int nv = EXACT == EN_EULER_WAVE ? DIM + 2 : (EXACT == EN_ADVECTION_WAVE ? 1 : nv_);
     constexpr int NA = 2 * N - 1, NL = cpow(N, DIM - 1), NN = cpow(N, DIM), NP = cpow(NA, DIM);
     extern __shared__ double dyn[];
     __shared__ double V[NA * N], wa[NA], red[4][18];
@@ -199,8 +217,6 @@ __global__ void __launch_bounds__(256) error_norms_kernel(const double* __restri
     double* const xa = dyn + (int64_t)wave * en_wave_doubles<DIM, N>(nv);
     double* const s1 = xa + DIM * NA;                              // [v][a0][line]
     double* const s2 = s1 + (DIM > 1 ? nv * NA * NL : 0);          // [v][a0][a1][k]
-    IcParams q = q0;
-    q.dim = DIM;
     double l2[9], li[9];
 #pragma unroll
     for (int v = 0; v < 9; ++v) l2[v] = li[v] = 0.0;
@@ -265,7 +281,26 @@ __global__ void __launch_bounds__(256) error_norms_kernel(const double* __restri
                 wq *= wa[ai[d]];
             }
             double uex[9];
-            initial_condition(q, x, t, 0, uex);
+            if constexpr (EXACT == EN_EULER_WAVE) {
+                double xs = 0.0;
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) xs += x[d];
+                const double ini = euler_wave(xs, t);
+#pragma unroll
+                for (int v = 0; v < 9; ++v) uex[v] = v == DIM + 1 ? ini * ini : ini;
+            } else if constexpr (EXACT == EN_ADVECTION_WAVE) {
+                double xs = 0.0;
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) xs += x[d] - q.a[d] * t;
+                const double w = advection_wave(xs);
+#pragma unroll
+                for (int v = 0; v < 9; ++v) uex[v] = w;
+            } else {
+                double ug[9];
+                initial_condition(q, x, t, 0, ug);
+#pragma unroll
+                for (int v = 0; v < 9; ++v) uex[v] = v < nv ? ug[v] : 0.0;
+            }
             const double* Vl = V + ai[DIM - 1] * N;
 #pragma unroll
             for (int v = 0; v < 9; ++v) {

@@ -157,6 +157,44 @@ static int scratch_ptr(double** out) {
 }
 
 // ---------------------------------------------------------------------------
+// Pinned result slots of the reductions.  Pinning a page takes milliseconds, so
+// contexts share one page of 64 slots (allocated with the first context, kept
+// until the process ends); a context takes a slot in create and gives it back
+// in destroy, and only contexts beyond 64 at a time pin memory of their own.
+// ---------------------------------------------------------------------------
+static constexpr int kResultDoubles = 32, kResultSlots = 64;
+static std::mutex g_result_mutex;
+static double* g_result_page = nullptr;
+static std::vector<int> g_result_free;
+
+static double* take_result_slot() {
+    std::lock_guard<std::mutex> lock(g_result_mutex);
+    const unsigned flags = hipHostMallocMapped | hipHostMallocPortable;
+    if (!g_result_page) {
+        if (hipHostMalloc((void**)&g_result_page, kResultSlots * kResultDoubles * sizeof(double), flags) != hipSuccess) {
+            g_result_page = nullptr;
+            return nullptr;
+        }
+        for (int q = kResultSlots - 1; q >= 0; --q) g_result_free.push_back(q);
+    }
+    if (!g_result_free.empty()) {
+        const int q = g_result_free.back();
+        g_result_free.pop_back();
+        return g_result_page + q * kResultDoubles;
+    }
+    double* p = nullptr;
+    return hipHostMalloc((void**)&p, kResultDoubles * sizeof(double), flags) == hipSuccess ? p : nullptr;
+}
+static void give_result_slot(double* p) {
+    if (!p) return;
+    std::lock_guard<std::mutex> lock(g_result_mutex);
+    if (p >= g_result_page && p < g_result_page + kResultSlots * kResultDoubles)
+        g_result_free.push_back((int)((p - g_result_page) / kResultDoubles));
+    else
+        (void)hipHostFree(p);
+}
+
+// ---------------------------------------------------------------------------
 // Lobatto-Legendre basis on the host (the matrices of
 // LobattoLegendreBasisGPU, reference basis_lobatto_legendre.jl:60-100).
 // Interior nodes: roots of P_{n-1} - P_{n+1} (proportional to (1-x^2) P_n'),
@@ -778,7 +816,7 @@ static void free_ctx(trixi_hip_ctx* c) {
                     c->d_mids, c->d_mori, c->d_mls, c->d_mnb, c->d_mflux};
     for (void* p : bufs)
         if (p) (void)hipFree(p);
-    if (c->h_result) (void)hipHostFree(c->h_result);
+    give_result_slot(c->h_result);
     delete c;
 }
 
@@ -1126,7 +1164,8 @@ int trixi_hip_create(const trixi_hip_config* config, const trixi_hip_mesh* mesh,
     ALLOC(c->d_time, 16 * sizeof(double));
     ALLOC(c->d_partial, (size_t)c->nblocks_red * 18 * sizeof(double));
     ALLOC(c->d_arrived, sizeof(unsigned));
-    if (hipHostMalloc((void**)&c->h_result, 32 * sizeof(double), hipHostMallocMapped) != hipSuccess)
+    c->h_result = take_result_slot();
+    if (!c->h_result)
         return cleanup_fail(TRIXI_HIP_ENOMEM, "hipHostMalloc failed for the reduction results");
     if (hipMemset(c->d_arrived, 0, sizeof(unsigned)) != hipSuccess)
         return cleanup_fail(TRIXI_HIP_EDEVICE, "hipMemset failed in create");
@@ -1625,9 +1664,18 @@ static hipError_t launch_error_norms(trixi_hip_ctx* ctx, const double* u, const 
     const size_t wave_bytes = en_wave_doubles<DIM, N>(ctx->nv) * sizeof(double);
     const int waves = wave_bytes * 4 <= 60 * 1024 ? 4 : (wave_bytes * 2 <= 60 * 1024 ? 2 : 1);
     const int blocks = (int)std::min<int64_t>((ctx->E + waves - 1) / waves, ctx->nblocks_red);
-    hipLaunchKernelGGL((error_norms_kernel<DIM, N>), dim3(blocks), dim3(64 * waves), (unsigned)(waves * wave_bytes), s,
-                       u, ctx->d_x, ctx->d_invJ, ctx->d_partial, ctx->h_result, ctx->d_arrived, ctx->d_Vdm, ctx->d_wa,
-                       ctx->E, q, t, ctx->nv);
+    const bool wave = q.ic == TRIXI_HIP_IC_CONVERGENCE_TEST;
+#define TRIXI_HIP_EN(X)                                                                                             \
+    hipLaunchKernelGGL((error_norms_kernel<DIM, N, X>), dim3(blocks), dim3(64 * waves), (unsigned)(waves * wave_bytes), \
+                       s, u, ctx->d_x, ctx->d_invJ, ctx->d_partial, ctx->h_result, ctx->d_arrived, ctx->d_Vdm,        \
+                       ctx->d_wa, ctx->E, q, t, ctx->nv)
+    if (wave && q.eq == EQ_EULER)
+        TRIXI_HIP_EN(EN_EULER_WAVE);
+    else if (wave && q.eq == EQ_LINADV)
+        TRIXI_HIP_EN(EN_ADVECTION_WAVE);
+    else
+        TRIXI_HIP_EN(EN_GENERAL);
+#undef TRIXI_HIP_EN
     return hipGetLastError();
 }
 
@@ -1666,10 +1714,22 @@ int trixi_hip_error_norms(trixi_hip_ctx* ctx, const double* u, int32_t ic, doubl
 int trixi_hip_integrate(trixi_hip_ctx* ctx, const double* u, double* integral, trixi_hip_stream stream) {
     if (!ctx || !u || !integral) return fail(TRIXI_HIP_EINVAL, "null argument");
     hipStream_t s = (hipStream_t)stream;
-#define IK(D)                                                                                                        \
-    hipLaunchKernelGGL((integrate_kernel<D>), dim3(reduction_blocks(ctx)), dim3(RED_THREADS), 0, s, u, ctx->d_invJ,    \
-                       ctx->d_partial, ctx->h_result, ctx->d_arrived, ctx->d_w, ctx->N, ctx->nn, ctx->E, ctx->nv)
-    if (ctx->dim == 1) IK(1); else if (ctx->dim == 2) IK(2); else IK(3);
+#define IK(D, NQ)                                                                                                  \
+    hipLaunchKernelGGL((integrate_kernel<D, NQ>), dim3(reduction_blocks(ctx)), dim3(RED_THREADS), 0, s, u, ctx->d_invJ, \
+                       ctx->d_partial, ctx->h_result, ctx->d_arrived, ctx->d_w, ctx->E, ctx->nv)
+#define IKN(NQ)                                                                    \
+    case NQ:                                                                       \
+        if (ctx->dim == 1) IK(1, NQ); else if (ctx->dim == 2) IK(2, NQ); else IK(3, NQ); \
+        break
+    switch (ctx->N) {
+        IKN(2);
+        IKN(3);
+        IKN(4);
+        IKN(5);
+        default:
+            return fail(TRIXI_HIP_EUNSUPPORTED, "integrals are built for polydeg 1 to 4");
+    }
+#undef IKN
 #undef IK
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s));
