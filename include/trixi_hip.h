@@ -333,6 +333,20 @@ int trixi_hip_max_dt(trixi_hip_ctx* ctx, const double* u, double* max_dt,
 int trixi_hip_max_dt_f32(trixi_hip_ctx* ctx, const float* u, double* max_dt,
                          trixi_hip_stream stream);
 
+/* Up to max_steps CarpenterKennedy2N54 steps of u in place from *t to t_end
+ * (k: the 2N register, its input ignored): steps of size cfl * max_dt(u) when
+ * cfl > 0, else of size dt, the last one shortened to end at t_end.  *t and
+ * *nsteps return the time reached and the steps taken; blocks until they are on
+ * the host, but not between the steps (max_dt, the stage times and the end of
+ * the run stay on the device).  Replaces the reference's solve loop with a
+ * StepsizeCallback (examples/euler_ec_3d.jl:45-55). */
+int trixi_hip_advance(trixi_hip_ctx* ctx, double* u, double* k, double* t, double t_end,
+                      double cfl, double dt, int64_t max_steps, int64_t* nsteps,
+                      trixi_hip_stream stream);
+int trixi_hip_advance_f32(trixi_hip_ctx* ctx, float* u, float* k, double* t, double t_end,
+                          double cfl, double dt, int64_t max_steps, int64_t* nsteps,
+                          trixi_hip_stream stream);
+
 /* trixi_hip_max_dt without any allocation: the block partials and the maximum
  * go to a static device scratch of 2048 doubles (16 KiB, held by every GPU
  * the library runs on until the process ends) instead of the context's

@@ -99,6 +99,8 @@ SIGNATURES = {
     "trixi_hip_sync": (ctypes.c_int, [_P]),
     "trixi_hip_max_dt": (ctypes.c_int, [_P, _P, _P, _P]),
     "trixi_hip_max_dt_f32": (ctypes.c_int, [_P, _P, _P, _P]),
+    "trixi_hip_advance": (ctypes.c_int, [_P, _P, _P, _P, _D, _D, _D, ctypes.c_int64, _P, _P]),
+    "trixi_hip_advance_f32": (ctypes.c_int, [_P, _P, _P, _P, _D, _D, _D, ctypes.c_int64, _P, _P]),
     "trixi_hip_max_dt_noalloc": (ctypes.c_int, [_P, _P, _P, _P]),
     "trixi_hip_error_norms": (ctypes.c_int, [_P, _P, _I32, _D, _U64, _P, _P, _P]),
     "trixi_hip_integrate": (ctypes.c_int, [_P, _P, _P, _P]),

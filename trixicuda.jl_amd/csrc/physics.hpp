@@ -230,17 +230,17 @@ __device__ __forceinline__ void log_free_means(double x1, double y1, double x2, 
     const double r1 = r * s2, r2 = r * s1;
     const double z1 = d1 * r1, z2 = d2 * r2;
     const double q1 = z1 * z1, q2 = z2 * z2;
-    double Q = fma(q1, fastlog_const(-0.008948152998574805), fastlog_const(-0.01088099532782093));
-    Q = fma(q1, Q, fastlog_const(-0.015097271029888403));
-    Q = fma(q1, Q, fastlog_const(-0.023280421147242054));
-    Q = fma(q1, Q, fastlog_const(-0.0444444444524844));
-    Q = fma(q1, Q, fastlog_const(-0.1666666666666553));
+    double Q = fma(q1, fastlog_const<true>(-0.008948152998574805), fastlog_const<true>(-0.01088099532782093));
+    Q = fma(q1, Q, fastlog_const<true>(-0.015097271029888403));
+    Q = fma(q1, Q, fastlog_const<true>(-0.023280421147242054));
+    Q = fma(q1, Q, fastlog_const<true>(-0.0444444444524844));
+    Q = fma(q1, Q, fastlog_const<true>(-0.1666666666666553));
     Q = fma(q1, Q, 0.5);
-    double Pq = fma(q2, fastlog_const(0.16481117002486795), fastlog_const(0.1814740093132822));
-    Pq = fma(q2, Pq, fastlog_const(0.2222275413776025));
-    Pq = fma(q2, Pq, fastlog_const(0.28571424363123693));
-    Pq = fma(q2, Pq, fastlog_const(0.4000000001583343));
-    Pq = fma(q2, Pq, fastlog_const(0.6666666666664435));
+    double Pq = fma(q2, fastlog_const<true>(0.16481117002486795), fastlog_const<true>(0.1814740093132822));
+    Pq = fma(q2, Pq, fastlog_const<true>(0.2222275413776025));
+    Pq = fma(q2, Pq, fastlog_const<true>(0.28571424363123693));
+    Pq = fma(q2, Pq, fastlog_const<true>(0.4000000001583343));
+    Pq = fma(q2, Pq, fastlog_const<true>(0.6666666666664435));
     Pq = fma(q2, Pq, 2.0);
     mean1 = s1 * Q;
     inv_mean2 = Pq * r2;
@@ -249,8 +249,8 @@ __device__ __forceinline__ void log_free_means(double x1, double y1, double x2, 
         const bool near1 = fabs(d1) < 0.15 * s1, near2 = fabs(d2) < 0.15 * s2;
         if (__builtin_amdgcn_ballot_w64(!(near1 && near2)) != 0) {
             const double nan = __builtin_nan("");
-            const double l1 = x1 > 0.0 ? fast_log(rdiv(y1, x1)) : nan;
-            const double l2 = x2 > 0.0 ? fast_log(rdiv(y2, x2)) : nan;
+            const double l1 = x1 > 0.0 ? fast_log<true>(rdiv(y1, x1)) : nan;
+            const double l2 = x2 > 0.0 ? fast_log<true>(rdiv(y2, x2)) : nan;
             mean1 = near1 ? mean1 : rdiv(d1, l1);
             inv_mean2 = near2 ? inv_mean2 : rdiv(l2, d2);
         }

@@ -29,16 +29,17 @@ __device__ __forceinline__ void store_partial(double* p, double x) {
 // the others their maximum) in the last block to arrive, which writes `out` and
 // leaves `arrived` at zero for the next call.  Every thread of every block calls
 // it after its block's store_partial calls.
+// Returns true in the last block's thread 0, with component 0 in `first`.
 template <int THREADS>
-__device__ __forceinline__ void finish_partials(const double* partial, double* out, unsigned* arrived, int m,
-                                                int nsum) {
+__device__ __forceinline__ bool finish_partials(const double* partial, double* out, unsigned* arrived, int m,
+                                                int nsum, double& first) {
     __shared__ bool last;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's partials have arrived
     __syncthreads();
     if (threadIdx.x == 0)
         last = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
     __syncthreads();
-    if (!last) return;
+    if (!last) return false;
     asm volatile("" ::: "memory");
     const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
     for (int c = wave; c < m; c += THREADS / 64) {
@@ -64,9 +65,66 @@ __device__ __forceinline__ void finish_partials(const double* partial, double* o
             x = sum ? x + y : fmax(x, y);
         }
         if (lane == 0) out[c] = x;
+        if (c == 0) first = x;
     }
     if (threadIdx.x == 0) __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return threadIdx.x == 0;
 }
+template <int THREADS>
+__device__ __forceinline__ void finish_partials(const double* partial, double* out, unsigned* arrived, int m,
+                                                int nsum) {
+    double first = 0.0;
+    finish_partials<THREADS>(partial, out, arrived, m, nsum, first);
+}
+
+// The time loop on the device: the stage times of the CarpenterKennedy2N54 step
+// from the current time, time = {stage time, dt} x 5, then {t, done}.  A step of
+// size h is shortened to end at t_end (select_step's rule, the same operations
+// in the same order); once t has reached t_end every further step sets `done`,
+// which the stages read.  log takes {t after the step, h}, h < 0 for no step.
+constexpr int TIME_T = 10, TIME_DONE = 11, TIME_DOUBLES = 16;
+struct StepControl {
+    double* time;  // nullptr: a reduction only
+    double* log;   // pinned
+    double t_end, cfl;
+    int N;
+    double c[5];
+};
+__device__ __forceinline__ void next_step(const StepControl& q, double h) {
+    // (no fused multiply-adds but the stage times', which set_time_kernel fuses:
+    // the times equal a host loop's bit for bit)
+#pragma clang fp contract(off)
+    const double t = q.time[TIME_T];
+    if (!(t < q.t_end)) {
+        q.time[TIME_DONE] = 1.0;
+        q.log[0] = t;
+        q.log[1] = -1.0;
+        return;
+    }
+    double tn = t + h;
+    if (tn >= q.t_end) {
+        h = q.t_end - t;
+        tn = q.t_end;
+    }
+    for (int s = 0; s < 5; ++s) {
+        q.time[2 * s] = fma(q.c[s], h, t);
+        q.time[2 * s + 1] = h;
+    }
+    q.time[TIME_T] = tn;
+    q.log[0] = tn;
+    q.log[1] = h;
+}
+// 2 / (N max) of the largest scaled wave speed
+__host__ __device__ inline double max_dt_of(int N, double m) {
+    const double tiny = 4.9406564584124654e-324;  // nextafter(0, 1)
+    if (!(m > tiny)) m = tiny;
+    return 2.0 / (N * m);
+}
+__global__ void start_time_kernel(double* time, double t) {
+    time[TIME_T] = t;
+    time[TIME_DONE] = 0.0;
+}
+__global__ void next_step_kernel(StepControl q, double dt) { next_step(q, dt); }
 
 // Elements per pass of a block and threads of the element reductions: 16
 // consecutive elements (whole 128-byte rows of an FP64 state) by 16 groups that
@@ -80,7 +138,7 @@ __global__ void __launch_bounds__(RED_THREADS) max_speed_kernel(const S* __restr
                                                                 const double* __restrict__ invJ,
                                                                 double* __restrict__ partial, double* out,
                                                                 unsigned* arrived, int nn, int64_t E,
-                                                                PhysParams phys) {
+                                                                PhysParams phys, StepControl step) {
     __shared__ double red[RED_THREADS / 64][DIM][RED_ELEMS];
     const PhysR<double> P = PhysR<double>::from(phys);
     const int c = threadIdx.x % RED_ELEMS, g = threadIdx.x / RED_ELEMS;
@@ -126,7 +184,11 @@ __global__ void __launch_bounds__(RED_THREADS) max_speed_kernel(const S* __restr
         for (int w = 8; w > 0; w >>= 1) best = fmax(best, __shfl_xor(best, w));
         if (threadIdx.x == 0) store_partial(&partial[blockIdx.x], best);
     }
-    finish_partials<RED_THREADS>(partial, out, arrived, 1, 0);
+    double m = 0.0;
+    if (finish_partials<RED_THREADS>(partial, out, arrived, 1, 0, m) && step.time != nullptr) {
+#pragma clang fp contract(off)
+        next_step(step, step.cfl * max_dt_of(step.N, m));
+    }
 }
 
 // Block sums of per-thread values into partial[blockIdx.x * m + c0 + v].

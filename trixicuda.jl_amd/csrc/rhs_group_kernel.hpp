@@ -176,6 +176,8 @@ __global__ void __launch_bounds__((group_threads<DIM, N, M>()), WAVES) rhs_group
     };
     if (faces) load_faces(0, um, up);
 
+    if (RK && a.done != nullptr && *a.done != 0.0) return;  // uniform
+
     // ---- node pass ---------------------------------------------------------
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {

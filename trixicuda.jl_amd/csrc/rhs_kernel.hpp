@@ -103,6 +103,7 @@ struct RhsArgs {
     void* k;                  // 2N register (RK mode)
     void* u_out;              // RK mode: u_out = u + b k
     const double* time;       // RK mode: device scalars {t, dt}
+    const double* done;       // RK mode, or nullptr: nonzero once the run has reached its end (nothing to do)
     const int32_t* nbr;       // [2*DIM][E] neighbour element per face (-x,+x,-y,+y,-z,+z)
     const double* invJ;       // [E]
     const double* alpha_raw;  // [E] HG blending factors before smoothing
@@ -390,6 +391,8 @@ rhs_kernel(const RhsArgs a) {
             up_next[v] = (double)U[soa(v, base0, np0, slab, E32)];
         }
     }
+
+    if (RK && a.done != nullptr && *a.done != 0.0) return;  // uniform
 
     // ---- node data, once per node: coalesced loads (element innermost) -----
     // Every lane visits NIT (node, element) pairs: NN * M / NT, rounded up.
@@ -943,6 +946,8 @@ rhs_np_kernel(const RhsArgs a) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) ub[v] = (R)U[soa(v, nn_face, nbe, slab, E32)];
     }
+
+    if (RK && a.done != nullptr && *a.done != 0.0) return;  // uniform
 
     if (last) {
         R uc[NV];

@@ -162,7 +162,8 @@ static int scratch_ptr(double** out) {
 // until the process ends); a context takes a slot in create and gives it back
 // in destroy, and only contexts beyond 64 at a time pin memory of their own.
 // ---------------------------------------------------------------------------
-static constexpr int kResultDoubles = 32, kResultSlots = 64;
+// (results of a reduction, then the log of up to kChunk steps of a time loop)
+static constexpr int kChunk = 32, kLog = 32, kResultDoubles = kLog + 2 * kChunk, kResultSlots = 64;
 static std::mutex g_result_mutex;
 static double* g_result_page = nullptr;
 static std::vector<int> g_result_free;
@@ -1161,7 +1162,7 @@ int trixi_hip_create(const trixi_hip_config* config, const trixi_hip_mesh* mesh,
     ALLOC(c->d_x, (size_t)dim * nn * E * sizeof(double));
     ALLOC(c->d_alpha_raw, E * sizeof(double));
     ALLOC(c->d_alpha, E * sizeof(double));
-    ALLOC(c->d_time, 16 * sizeof(double));
+    ALLOC(c->d_time, TIME_DOUBLES * sizeof(double));
     ALLOC(c->d_partial, (size_t)c->nblocks_red * 18 * sizeof(double));
     ALLOC(c->d_arrived, sizeof(unsigned));
     c->h_result = take_result_slot();
@@ -1429,7 +1430,7 @@ int trixi_hip_compute_coefficients(trixi_hip_ctx* ctx, double* u, int32_t ic, do
 // it cannot update in place: stage 0 reads u and writes buffer A, then the
 // stages alternate A -> B -> A -> B, and stage 4 reads B and writes the
 // caller's u, which no stage after 0 reads.
-static int enqueue_rk_stages(trixi_hip_ctx* c, void* u, void* k, hipStream_t s) {
+static int enqueue_rk_stages(trixi_hip_ctx* c, void* u, void* k, hipStream_t s, const double* done = nullptr) {
     // two stage buffers of the context's state type in d_tmp
     const size_t bytes = (size_t)c->nvalues * (fp32_state(c) ? sizeof(float) : sizeof(double));
     void* bufA = c->d_tmp;
@@ -1457,6 +1458,7 @@ static int enqueue_rk_stages(trixi_hip_ctx* c, void* u, void* k, hipStream_t s) 
         a.k = k;
         a.u_out = nxt;
         a.time = c->d_time + 2 * st;
+        a.done = done;
         a.rk_a = CK_A[st];
         a.rk_b = CK_B[st];
         a.rk_first = (st == 0);
@@ -1569,12 +1571,12 @@ static int reduction_blocks(const trixi_hip_ctx* c) {
 // doubles) and the arrival count in `arrived` (zero before and after).
 extern "C++" template <typename S>
 static int launch_max_speed(trixi_hip_ctx* ctx, const S* u, hipStream_t s, int blocks, double* partial,
-                            double* result, unsigned* arrived) {
+                            double* result, unsigned* arrived, const StepControl& step = StepControl{}) {
     const PhysParams& P = ctx->args.phys;
     const int eq = ctx->cfg.equation, dim = ctx->dim;
 #define MS(EQT, D)                                                                                                 \
     hipLaunchKernelGGL((max_speed_kernel<EQT, D, S>), dim3(blocks), dim3(RED_THREADS), 0, s, u, ctx->d_invJ, partial, \
-                       result, arrived, ctx->nn, ctx->E, P)
+                       result, arrived, ctx->nn, ctx->E, P, step)
     if (eq == TRIXI_HIP_LINEAR_SCALAR_ADVECTION) {
         if (dim == 1) MS(LinAdv<1>, 1); else if (dim == 2) MS(LinAdv<2>, 2); else MS(LinAdv<3>, 3);
     } else if (eq == TRIXI_HIP_COMPRESSIBLE_EULER) {
@@ -1606,18 +1608,12 @@ static int launch_max_speed(trixi_hip_ctx* ctx, const S* u, hipStream_t s, int b
     return TRIXI_HIP_OK;
 }
 
-static double max_dt_of(const trixi_hip_ctx* ctx, double m) {
-    const double tiny = nextafter(0.0, 1.0);
-    if (!(m > tiny)) m = tiny;
-    return 2.0 / (ctx->N * m);
-}
-
 extern "C++" template <typename S>
 static int max_dt_any(trixi_hip_ctx* ctx, const S* u, double* max_dt, hipStream_t s) {
     int rc = launch_max_speed(ctx, u, s, reduction_blocks(ctx), ctx->d_partial, ctx->h_result, ctx->d_arrived);
     if (rc) return rc;
     HIP_TRY(hipStreamSynchronize(s));
-    *max_dt = max_dt_of(ctx, ctx->h_result[0]);
+    *max_dt = max_dt_of(ctx->N, ctx->h_result[0]);
     return TRIXI_HIP_OK;
 }
 
@@ -1654,8 +1650,84 @@ int trixi_hip_max_dt_noalloc(trixi_hip_ctx* ctx, const double* u, double* max_dt
     double m = 0.0;
     HIP_TRY(hipMemcpyAsync(&m, result, sizeof(double), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
-    *max_dt = max_dt_of(ctx, m);
+    *max_dt = max_dt_of(ctx->N, m);
     return TRIXI_HIP_OK;
+}
+
+// Up to max_steps CarpenterKennedy2N54 steps from *t, without a host
+// synchronisation per step: the wave-speed reduction (or, with a fixed dt, a
+// kernel of one thread) leaves the step's times on the device for the stages and
+// logs the step in pinned memory; the host queues a chunk of steps, waits once
+// and reads the log.  A step past the end does nothing (RhsArgs::done), so a
+// chunk may be longer than what is left.
+extern "C++" template <typename S>
+static int advance_any(trixi_hip_ctx* c, S* u, S* k, double* t, double t_end, double cfl, double dt,
+                       int64_t max_steps, int64_t* nsteps, hipStream_t s) {
+    StepControl q{};
+    q.time = c->d_time;
+    q.t_end = t_end;
+    q.cfl = cfl;
+    q.N = c->N;
+    for (int st = 0; st < 5; ++st) q.c[st] = CK_C[st];
+    hipLaunchKernelGGL(start_time_kernel, dim3(1), dim3(1), 0, s, c->d_time, *t);
+    HIP_TRY(hipGetLastError());
+    double h = cfl > 0.0 ? 0.0 : dt;  // last step size: how many steps are left at most a guess
+    int64_t done = 0;
+    while (*t < t_end && done < max_steps) {
+        // by the last step size, two where there is none yet
+        const double left = h > 0.0 ? ceil((t_end - *t) / h) : 2.0;
+        int64_t chunk = std::min<int64_t>(kChunk, max_steps - done);
+        if (left < (double)chunk) chunk = left > 1.0 ? (int64_t)left : 1;
+        for (int64_t i = 0; i < chunk; ++i) {
+            q.log = c->h_result + kLog + 2 * i;
+            if (cfl > 0.0) {
+                int rc = launch_max_speed(c, (const S*)u, s, reduction_blocks(c), c->d_partial, c->h_result,
+                                          c->d_arrived, q);
+                if (rc) return rc;
+            } else {
+                hipLaunchKernelGGL(next_step_kernel, dim3(1), dim3(1), 0, s, q, dt);
+                HIP_TRY(hipGetLastError());
+            }
+            int rc = enqueue_rk_stages(c, u, k, s, c->d_time + TIME_DONE);
+            if (rc) return rc;
+        }
+        HIP_TRY(hipStreamSynchronize(s));
+        for (int64_t i = 0; i < chunk; ++i) {
+            const double* log = c->h_result + kLog + 2 * i;
+            if (log[1] < 0.0) break;
+            *t = log[0];
+            h = log[1];
+            ++done;
+            *nsteps = done;
+        }
+    }
+    return TRIXI_HIP_OK;
+}
+
+static int check_advance(const trixi_hip_ctx* c, const void* u, const void* k, const double* t, double cfl, double dt,
+                         const int64_t* nsteps) {
+    if (!c || !u || !k || !t || !nsteps) return fail(TRIXI_HIP_EINVAL, "null argument");
+    if (u == k) return fail(TRIXI_HIP_EINVAL, "u and k must be distinct");
+    if (!(cfl > 0.0) && !(dt > 0.0)) return fail(TRIXI_HIP_EINVAL, "advance needs a positive cfl or a positive dt");
+    return TRIXI_HIP_OK;
+}
+
+int trixi_hip_advance(trixi_hip_ctx* ctx, double* u, double* k, double* t, double t_end, double cfl, double dt,
+                      int64_t max_steps, int64_t* nsteps, trixi_hip_stream stream) {
+    int rc = check_advance(ctx, u, k, t, cfl, dt, nsteps);
+    if (rc) return rc;
+    if (fp32_state(ctx)) return fail(TRIXI_HIP_EINVAL, "this context's state is FP32: use trixi_hip_advance_f32");
+    *nsteps = 0;
+    return advance_any(ctx, u, k, t, t_end, cfl, dt, max_steps, nsteps, (hipStream_t)stream);
+}
+
+int trixi_hip_advance_f32(trixi_hip_ctx* ctx, float* u, float* k, double* t, double t_end, double cfl, double dt,
+                          int64_t max_steps, int64_t* nsteps, trixi_hip_stream stream) {
+    int rc = check_advance(ctx, u, k, t, cfl, dt, nsteps);
+    if (rc) return rc;
+    if (!fp32_state(ctx)) return fail(TRIXI_HIP_EINVAL, "this context's state is FP64: use trixi_hip_advance");
+    *nsteps = 0;
+    return advance_any(ctx, u, k, t, t_end, cfl, dt, max_steps, nsteps, (hipStream_t)stream);
 }
 
 extern "C++" template <int DIM, int N>

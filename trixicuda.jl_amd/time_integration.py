@@ -71,6 +71,22 @@ def select_step(t, h, t1, save_times=()):
     return end - t, end
 
 
+def advance(u, k, t, t_end, semi, cfl=0.0, dt=0.0, max_steps=10**7, stream=None):
+    """Up to max_steps CK2N54 steps of u in place from t to t_end, of size
+    cfl * max_dt(u) (cfl > 0) or dt, without a synchronisation per step.
+    Returns (t, number of steps)."""
+    import ctypes
+    import torch
+    semi.check_vector(u, "u")
+    semi.check_vector(k, "k")
+    s = stream if stream is not None else torch.cuda.current_stream()
+    tt, n = ctypes.c_double(t), ctypes.c_int64()
+    fn = L.lib().trixi_hip_advance_f32 if semi.fp32_state else L.lib().trixi_hip_advance
+    L.check(fn(semi.ctx, _ptr(u), _ptr(k), ctypes.byref(tt), float(t_end), float(cfl), float(dt), int(max_steps),
+               ctypes.byref(n), ctypes.c_void_p(s.cuda_stream)))
+    return tt.value, n.value
+
+
 def solve(ode, alg=None, dt=None, callback=(), use_graph=True, maxiters=10**7):
     """Integrate ode over its tspan; returns a Solution with the final state."""
     import torch
@@ -89,7 +105,19 @@ def solve(ode, alg=None, dt=None, callback=(), use_graph=True, maxiters=10**7):
     stream = torch.cuda.Stream()
     stream.wait_stream(torch.cuda.current_stream())
     t, nsteps, h = t0, 0, 0.0
+    # steps without host work between them run as one native loop: nothing to
+    # save, and analysis only at known step numbers
+    cfl = stepsize.cfl if type(stepsize) is StepsizeCallback else 0.0
+    native = not saves and all(type(a) is AnalysisCallback for a in analysis) and (
+        cfl > 0.0 if stepsize is not None else dt > 0.0)
     with torch.cuda.stream(stream):
+        while native and t < t1 and nsteps < maxiters:
+            todo = min([maxiters - nsteps] + [a.interval - nsteps % a.interval for a in analysis if a.interval > 0])
+            t, n = advance(u, k, t, t1, semi, cfl=cfl, dt=0.0 if stepsize is not None else dt, max_steps=todo,
+                           stream=stream)
+            nsteps += n
+            for a in analysis:
+                a(u, t, nsteps)
         for c in saves:
             c.initialize(u, t, stepsize.dt(u, semi) if stepsize is not None else dt, semi)
         while t < t1 and nsteps < maxiters:
