@@ -42,6 +42,12 @@ constexpr bool group_eligible() {
 template <int DIM, int N, class EQ, int VOL, int VF, int SF, int FVF, typename R, int M, bool RK, bool EXT = false,
           typename L = double, typename S = double>
 hipError_t launch_rhs(const RhsArgs& a, hipStream_t stream) {
+    auto consts = [&]() -> RhsConstArg<R> {
+        if constexpr (std::is_same<R, double>::value)
+            return a.consts;
+        else
+            return *a.host_consts;
+    };
     auto grid = [&](int m) {
         int64_t blocks = (a.E + m - 1) / m;
         if (a.nxcd > 1) blocks = (blocks + a.nxcd - 1) / a.nxcd * a.nxcd;
@@ -51,7 +57,7 @@ hipError_t launch_rhs(const RhsArgs& a, hipStream_t stream) {
         if (a.np) {
             constexpr int MN = np_elems<DIM, N>();
             hipLaunchKernelGGL((rhs_np_kernel<DIM, N, EQ, VOL, VF, SF, FVF, R, RK, L, S>), grid(MN),
-                               dim3(MN * cpow(N, DIM) * DIM), 0, stream, a);
+                               dim3(MN * cpow(N, DIM) * DIM), 0, stream, a, consts());
             return hipGetLastError();
         }
     }
@@ -62,10 +68,10 @@ hipError_t launch_rhs(const RhsArgs& a, hipStream_t stream) {
         constexpr int MG = EXT && (ME / 2 * cpow(N, DIM - 1)) % 64 == 0 ? ME / 2 : ME;
         constexpr int W = EQ::NV > 5 || EXT ? 2 : (DIM == 3 ? 4 : TRIXI_HIP_GROUP_WAVES2D);
         hipLaunchKernelGGL((rhs_group_kernel<DIM, N, EQ, VOL, VF, SF, FVF, MG, RK, EXT, W>), grid(MG),
-                           dim3(group_threads<DIM, N, MG>()), 0, stream, a);
+                           dim3(group_threads<DIM, N, MG>()), 0, stream, a, a.consts);
     } else {
         hipLaunchKernelGGL((rhs_kernel<DIM, N, EQ, VOL, VF, SF, FVF, R, M, RK, EXT, L, S>), grid(M),
-                           dim3(rhs_threads<DIM, N, M, R, RK, EQ::NV>()), 0, stream, a);
+                           dim3(rhs_threads<DIM, N, M, R, RK, EQ::NV>()), 0, stream, a, consts());
     }
     return hipGetLastError();
 }

@@ -94,7 +94,8 @@ __host__ __device__ constexpr int group_threads() {
 
 // WAVES: waves per SIMD the registers are allocated for
 template <int DIM, int N, class EQ, int VOL, int VF, int SF, int FVF, int M, bool RK, bool EXT, int WAVES>
-__global__ void __launch_bounds__((group_threads<DIM, N, M>()), WAVES) rhs_group_kernel(const RhsArgs a) {
+__global__ void __launch_bounds__((group_threads<DIM, N, M>()), WAVES) rhs_group_kernel(const RhsArgs a, const RhsConst* __restrict__ consts) {
+    const RhsConst& kc = *consts;
     constexpr int NL = cpow(N, DIM - 1);
     constexpr int NN = cpow(N, DIM);
     constexpr int GL = M * NL;                   // lanes of a group
@@ -127,7 +128,7 @@ __global__ void __launch_bounds__((group_threads<DIM, N, M>()), WAVES) rhs_group
     const int64_t e0 = xcd_tile(a.nxcd) * M;
     if (e0 >= E) return;  // whole workgroup: padding tile of the XCD mapping
     const int64_t ec = e0 + el < E ? e0 + el : E - 1;
-    const PhysR<double> P = PhysR<double>::from(a.phys);
+    const PhysR<double> P = PhysR<double>::from(kc.phys);
     double tnow = 0.0;
     if constexpr (EXT) tnow = RK ? a.time[0] : a.t_host;
 
@@ -209,20 +210,20 @@ __global__ void __launch_bounds__((group_threads<DIM, N, M>()), WAVES) rhs_group
         bool blended = false;
         if constexpr (VOL == VI_HG) {
             alpha = a.alpha_raw[ec];
-            if (a.smooth) {
+            if (kc.smooth) {
 #pragma unroll
                 for (int f = 0; f < 2 * DIM; ++f) {
                     if (EXT && nb[f] < 0) {
                         if (nb[f] == -1) continue;  // boundary: no neighbour
-                        const int32_t* mn = a.mnb + (int64_t)(-2 - nb[f]) * a.mK;
-                        for (int k = 0; k < a.mK; ++k)
+                        const int32_t* mn = kc.mnb + (int64_t)(-2 - nb[f]) * kc.mK;
+                        for (int k = 0; k < kc.mK; ++k)
                             if (mn[k] >= 0) alpha = dmax(alpha, 0.5 * a.alpha_raw[mn[k]]);
                         continue;
                     }
                     alpha = dmax(alpha, 0.5 * a.alpha_raw[nb[f]]);
                 }
             }
-            blended = !(fabs(alpha) <= a.atol);
+            blended = !(fabs(alpha) <= kc.atol);
             dg = blended ? 1.0 - alpha : 1.0;
         }
         Node nd[N];
@@ -245,8 +246,8 @@ __global__ void __launch_bounds__((group_threads<DIM, N, M>()), WAVES) rhs_group
             for (int j = i + 1; j < N; ++j) {
                 double f[NV];
                 node_flux<EQ, VF, TW, MEANS_NEAR, double, double>(nd[i], nullptr, nd[j], nullptr, 0, P, f);
-                const double fa = VOL == VI_HG ? dg * a.Ds[i * N + j] : a.Ds[i * N + j];
-                const double fb = VOL == VI_HG ? dg * a.Ds[j * N + i] : a.Ds[j * N + i];
+                const double fa = VOL == VI_HG ? dg * kc.Ds[i * N + j] : kc.Ds[i * N + j];
+                const double fb = VOL == VI_HG ? dg * kc.Ds[j * N + i] : kc.Ds[j * N + i];
 #pragma unroll
                 for (int v = 0; v < NV; ++v) {
                     al[i][v] += fa * f[v];
@@ -265,7 +266,7 @@ __global__ void __launch_bounds__((group_threads<DIM, N, M>()), WAVES) rhs_group
                     double f[NV];
                     node_flux<EQ, VF, TW, MEANS_ANY, double, double>(staged(base + i * s, o), nullptr,
                                                                      staged(base + j * s, o), nullptr, 0, P, f);
-                    const double fa = dg * a.Ds[i * N + j], fb = dg * a.Ds[j * N + i];
+                    const double fa = dg * kc.Ds[i * N + j], fb = dg * kc.Ds[j * N + i];
 #pragma unroll
                     for (int p = 0; p < N; ++p) {
                         const double w = p == i ? fa : (p == j ? fb : 0.0);
@@ -278,7 +279,7 @@ __global__ void __launch_bounds__((group_threads<DIM, N, M>()), WAVES) rhs_group
 #pragma unroll
             for (int p = 0; p < N; ++p) nd[p] = staged(base + p * s, o);
         }
-        if constexpr (EQ::NONCONS) line_noncons<N>(nd, a.Ds, (TW ? 1.0 : 0.5) * dg, al);
+        if constexpr (EQ::NONCONS) line_noncons<N>(nd, kc.Ds, (TW ? 1.0 : 0.5) * dg, al);
         if (VOL == VI_HG && blended) {
 #pragma unroll
             for (int p = 0; p + 1 < N; ++p) {
@@ -291,7 +292,7 @@ __global__ void __launch_bounds__((group_threads<DIM, N, M>()), WAVES) rhs_group
                     }
                 }
                 node_flux<EQ, FVF, TW, MEANS_ANY, double, double>(nd[p], ul, nd[p + 1], ur, 0, P, F);
-                const double wl = alpha * a.invw[p], wr = alpha * a.invw[p + 1];
+                const double wl = alpha * kc.invw[p], wr = alpha * kc.invw[p + 1];
                 if constexpr (EQ::NONCONS) {
                     // the left node takes f + nc(u_l, u_r)/2, the right f + nc(u_r, u_l)/2
                     constexpr double h = TW ? 1.0 : 0.5;
@@ -338,7 +339,7 @@ __global__ void __launch_bounds__((group_threads<DIM, N, M>()), WAVES) rhs_group
                     nm = o == f ? nb[2 * f] : nm;
                     np = o == f ? nb[2 * f + 1] : np;
                 }
-                if (a.bc) {
+                if (kc.bc) {
                     // outflow and slip walls read the inner state (mc, pc hold
                     // it: this element's own face node on the other end is not
                     // it, so it is read here)
@@ -347,14 +348,14 @@ __global__ void __launch_bounds__((group_threads<DIM, N, M>()), WAVES) rhs_group
                         for (int v = 0; v < NV; ++v) x[v] = U[soa(Rot::variable(v, o), node, ec, slab, E32)];
                     };
                     auto boundary = [&](int face, int node, double* x) {
-                        if ((a.outflow >> face) & 1) {
+                        if ((kc.outflow >> face) & 1) {
                             inner(node, x);
-                        } else if (a.bc == TRIXI_HIP_BC_SLIP_WALL) {
+                        } else if (kc.bc == TRIXI_HIP_BC_SLIP_WALL) {
                             inner(node, x);
                             x[1] = -x[1];
                         } else {
                             double b[NV];
-                            boundary_state<DIM, NN, NV, double>(a, ec, node, tnow, b);
+                            boundary_state<DIM, NN, NV, double>(a, kc, ec, node, tnow, b);
 #pragma unroll
                             for (int v = 0; v < NV; ++v) {
                                 const int w = Rot::variable(v, o);
@@ -403,12 +404,12 @@ __global__ void __launch_bounds__((group_threads<DIM, N, M>()), WAVES) rhs_group
                 }
                 constexpr double h = TW ? 2.0 : 1.0;
                 if (nm <= -2) {
-                    const double* mf = a.mflux + ((int64_t)(-2 - nm) * NL + line) * NV;
+                    const double* mf = kc.mflux + ((int64_t)(-2 - nm) * NL + line) * NV;
 #pragma unroll
                     for (int v = 0; v < NV; ++v) fm[v] = h * mf[Rot::variable(v, o)];
                 }
                 if (np <= -2) {
-                    const double* mf = a.mflux + ((int64_t)(-2 - np) * NL + line) * NV;
+                    const double* mf = kc.mflux + ((int64_t)(-2 - np) * NL + line) * NV;
 #pragma unroll
                     for (int v = 0; v < NV; ++v) fp[v] = h * mf[Rot::variable(v, o)];
                 }
@@ -416,8 +417,8 @@ __global__ void __launch_bounds__((group_threads<DIM, N, M>()), WAVES) rhs_group
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
                 const int w = Rot::variable(v, o);
-                fcs[(((2 * o) * NL + line) * NV + w) * M + el] = -a.lhat_m * fm[v];
-                fcs[(((2 * o + 1) * NL + line) * NV + w) * M + el] = a.lhat_p * fp[v];
+                fcs[(((2 * o) * NL + line) * NV + w) * M + el] = -kc.lhat_m * fm[v];
+                fcs[(((2 * o + 1) * NL + line) * NV + w) * M + el] = kc.lhat_p * fp[v];
             }
         }
     }
@@ -497,7 +498,7 @@ __global__ void __launch_bounds__((group_threads<DIM, N, M>()), WAVES) rhs_group
         double sv[NV];
 #pragma unroll
         for (int v = 0; v < NV; ++v) sv[v] = 0.0;
-        if (EXT && a.src) source_at<DIM, NN, NV>(a, e, n, tnow, sv);
+        if (EXT && kc.src) source_at<DIM, NN, NV>(a, kc, e, n, tnow, sv);
         double t_dt = 0.0;
         if (RK) t_dt = a.time[1];
 #pragma unroll

@@ -95,6 +95,43 @@ constexpr int MAXN = 8;
 #define TRIXI_HIP_PAR_DIRS_RK 1
 #endif
 
+// What a context's launches have in common, kept on the device: as kernel
+// arguments these 1.5 KB made a launch 4.2 us of host time instead of 2.9, which
+// bounds small meshes.
+struct RhsConst {
+    PhysParams phys;
+    double Ds[MAXN * MAXN];   // derivative_split (row-major)
+    double Dhat[MAXN * MAXN]; // derivative_dhat (row-major)
+    double invw[MAXN];        // inverse weights
+    double lhat_m, lhat_p;    // boundary_interpolation[1,1], [N,2]
+    double atol;              // HG pure-DG threshold
+    int smooth;               // HG smoothing
+    // non-periodic meshes and source terms
+    const double* x;          // node coordinates x[(d*NN + node)*E + e]
+    IcParams bc_ic;           // Dirichlet boundary state (faces with nbr < 0)
+    int bc;                   // enum trixi_hip_boundary_condition
+    int src;                  // enum trixi_hip_source_terms
+    int outflow;              // bit f: boundary face direction f takes the inner state
+    // L2 mortars: a face with nbr = -2 - slot takes its surface flux from
+    // mflux[(slot*NL + face node)*NV + v]; mnb[slot*mK + k] lists the elements
+    // across that face (-1 padded) for the blending-factor smoothing
+    const double* mflux;
+    const int32_t* mnb;
+    int mK;
+    // shock capturing: the indicator's inverse Vandermonde and parameters
+    const double* Vinv;
+    double ind_threshold, ind_s, ind_alpha_min, ind_alpha_max;
+    int ind_var;
+};
+
+// How a kernel takes them: by address with FP64 arithmetic; by value with FP32
+// arithmetic, whose roundings (which of two products a sum is fused with)
+// change with the form.
+template <typename R>
+using RhsConstArg = std::conditional_t<std::is_same<R, double>::value, const RhsConst* __restrict__, RhsConst>;
+__device__ __forceinline__ const RhsConst& consts_of(const RhsConst* p) { return *p; }
+__device__ __forceinline__ const RhsConst& consts_of(const RhsConst& v) { return v; }
+
 struct RhsArgs {
     // state vectors of the kernel's state type S (double, or float for the
     // FP32-state precision)
@@ -107,51 +144,29 @@ struct RhsArgs {
     const int32_t* nbr;       // [2*DIM][E] neighbour element per face (-x,+x,-y,+y,-z,+z)
     const double* invJ;       // [E]
     const double* alpha_raw;  // [E] HG blending factors before smoothing
-    int64_t E;
-    PhysParams phys;
-    double Ds[MAXN * MAXN];   // derivative_split (row-major)
-    double Dhat[MAXN * MAXN]; // derivative_dhat (row-major)
-    double invw[MAXN];        // inverse weights
-    double lhat_m, lhat_p;    // boundary_interpolation[1,1], [N,2]
-    double atol;              // HG pure-DG threshold
-    int smooth;               // HG smoothing
-    double rk_a, rk_b;        // RK stage coefficients (rk_a unused when rk_first)
-    int rk_first;
-    int nxcd;                 // XCDs the dispatcher deals workgroups to round robin
-    // non-periodic meshes and source terms
-    const double* x;          // node coordinates x[(d*NN + node)*E + e]
-    IcParams bc_ic;           // Dirichlet boundary state (faces with nbr < 0)
-    int bc;                   // enum trixi_hip_boundary_condition
-    int src;                  // enum trixi_hip_source_terms
-    int outflow;              // bit f: boundary face direction f takes the inner state
-    double t_host;            // rhs mode: time t
-    // L2 mortars: a face with nbr = -2 - slot takes its surface flux from
-    // mflux[(slot*NL + face node)*NV + v]; mnb[slot*mK + k] lists the elements
-    // across that face (-1 padded) for the blending-factor smoothing
-    const double* mflux;
-    const int32_t* mnb;
-    int mK;
-    // node-parallel form (small periodic conforming meshes, chosen on the host)
-    int np;
     // fused RK stage of the node-parallel form with shock capturing
     // (compressible Euler): the raw blending factors of u_out, the next
-    // stage's input, go to alpha_next (nullptr: not computed), with the
-    // indicator's inverse Vandermonde and parameters
+    // stage's input, go here (nullptr: not computed)
     double* alpha_next;
-    const double* Vinv;
-    double ind_threshold, ind_s, ind_alpha_min, ind_alpha_max;
-    int ind_var;
+    const RhsConst* consts;   // on the device, and the host's copy
+    const RhsConst* host_consts;
+    int64_t E;
+    double rk_a, rk_b;        // RK stage coefficients (rk_a unused when rk_first)
+    double t_host;            // rhs mode: time t
+    int rk_first;
+    int nxcd;                 // XCDs the dispatcher deals workgroups to round robin
+    int np;                   // host: node-parallel form (small periodic conforming meshes)
 };
 
 // Dirichlet state boundary_ic(x, t) at node `node` of element e (its face
 // node on a boundary face), in R.
 template <int DIM, int NN, int NV, typename R>
-__device__ __forceinline__ void boundary_state(const RhsArgs& a, int64_t e, int node, double t, R* ub) {
+__device__ __forceinline__ void boundary_state(const RhsArgs& a, const RhsConst& kc, int64_t e, int node, double t, R* ub) {
     double xx[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-    for (int d = 0; d < DIM; ++d) xx[d] = a.x[((int64_t)d * NN + node) * a.E + e];
+    for (int d = 0; d < DIM; ++d) xx[d] = kc.x[((int64_t)d * NN + node) * a.E + e];
     double uu[5];
-    boundary_value(a.bc_ic, xx, t, uu);
+    boundary_value(kc.bc_ic, xx, t, uu);
 #pragma unroll
     for (int v = 0; v < NV; ++v) ub[v] = (R)uu[v];
 }
@@ -160,34 +175,34 @@ __device__ __forceinline__ void boundary_state(const RhsArgs& a, int64_t e, int 
 // (compressible Euler, or the inviscid Burgers equation: the only scalar
 // equation built with source terms).
 template <int DIM, int NN, int NV>
-__device__ __forceinline__ void source_at(const RhsArgs& a, int64_t e, int node, double t, double* sv) {
+__device__ __forceinline__ void source_at(const RhsArgs& a, const RhsConst& kc, int64_t e, int node, double t, double* sv) {
     double xx[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-    for (int d = 0; d < DIM; ++d) xx[d] = a.x[((int64_t)d * NN + node) * a.E + e];
+    for (int d = 0; d < DIM; ++d) xx[d] = kc.x[((int64_t)d * NN + node) * a.E + e];
     if constexpr (NV == 1) {
         sv[0] = source_burgers_convergence_test(xx[0], t);
         return;
     }
-    if (a.src == TRIXI_HIP_SOURCE_POISSON_NONPERIODIC || a.src == TRIXI_HIP_SOURCE_HARMONIC) {
+    if (kc.src == TRIXI_HIP_SOURCE_POISSON_NONPERIODIC || kc.src == TRIXI_HIP_SOURCE_HARMONIC) {
         // hyperbolic diffusion: the relaxation -q / T_r reads this node's q
         double qv[3] = {0.0, 0.0, 0.0};
 #pragma unroll
         for (int d = 0; d < DIM; ++d) qv[d] = static_cast<const double*>(a.u)[((int64_t)(1 + d) * NN + node) * a.E + e];
         double s4[4];
-        source_hypdiff(DIM, a.src, a.phys.nu, a.phys.inv_Tr, xx, qv, s4);
+        source_hypdiff(DIM, kc.src, kc.phys.nu, kc.phys.inv_Tr, xx, qv, s4);
 #pragma unroll
         for (int v = 0; v < NV && v < 4; ++v) sv[v] = s4[v];
         return;
     }
     double s5[5];
-    if (a.bc_ic.eq == EQ_SHALLOW_WATER)
-        source_shallow_water_convergence_test(a.phys.grav, xx, t, s5);
-    else if (a.bc_ic.eq == EQ_EULER_QUASI1D)
-        source_quasi1d_convergence_test(a.phys.gamma, xx, t, s5);
-    else if (a.src == TRIXI_HIP_SOURCE_EOC_TEST_EULER)
-        source_eoc_test_euler(DIM, a.phys.gm1, xx, t, s5);
+    if (kc.bc_ic.eq == EQ_SHALLOW_WATER)
+        source_shallow_water_convergence_test(kc.phys.grav, xx, t, s5);
+    else if (kc.bc_ic.eq == EQ_EULER_QUASI1D)
+        source_quasi1d_convergence_test(kc.phys.gamma, xx, t, s5);
+    else if (kc.src == TRIXI_HIP_SOURCE_EOC_TEST_EULER)
+        source_eoc_test_euler(DIM, kc.phys.gm1, xx, t, s5);
     else
-        source_convergence_test(DIM, a.phys.gm1, xx, t, s5);
+        source_convergence_test(DIM, kc.phys.gm1, xx, t, s5);
 #pragma unroll
     for (int v = 0; v < NV; ++v) sv[v] = s5[v];
 }
@@ -247,7 +262,8 @@ __host__ __device__ constexpr int rhs_threads() {
 template <int DIM, int N, class EQ, int VOL, int VF, int SF, int FVF, typename R, int M, bool RK, bool EXT,
           typename L, typename S>
 __global__ void __launch_bounds__((rhs_threads<DIM, N, M, R, RK, EQ::NV>()), TRIXI_HIP_MIN_WAVES)
-rhs_kernel(const RhsArgs a) {
+rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
+    const RhsConst& kc = consts_of(consts);
     static_assert(!EXT || std::is_same<S, double>::value, "boundaries, mortars and sources take FP64 states");
     const S* __restrict__ U = static_cast<const S*>(a.u);
     S* __restrict__ DU = static_cast<S*>(a.du);
@@ -303,7 +319,7 @@ rhs_kernel(const RhsArgs a) {
     const int64_t e = e0 + el;
     const bool valid = e < E;
     const int64_t ec = valid ? e : E - 1;
-    const PhysR<R> P = PhysR<R>::from(a.phys);
+    const PhysR<R> P = PhysR<R>::from(kc.phys);
 
     // Face neighbours of all 2*DIM faces, and the neighbour face data of the
     // first direction, are requested before the node pass so that their
@@ -438,15 +454,15 @@ rhs_kernel(const RhsArgs a) {
     bool dg_only = true;
     if (VOL == VI_HG) {
         double al = a.alpha_raw[ec];
-        if (a.smooth) {
+        if (kc.smooth) {
 #pragma unroll
             for (int s = 0; s < 2 * DIM; ++s) {
                 if (EXT && nb[s] < 0) {
                     // boundary faces have no neighbour; a mortar face has the
                     // elements on the other side of the mortar
                     if (nb[s] == -1) continue;
-                    const int32_t* mn = a.mnb + (int64_t)(-2 - nb[s]) * a.mK;
-                    for (int k = 0; k < a.mK; ++k) {
+                    const int32_t* mn = kc.mnb + (int64_t)(-2 - nb[s]) * kc.mK;
+                    for (int k = 0; k < kc.mK; ++k) {
                         if (mn[k] < 0) continue;
                         const double an = 0.5 * a.alpha_raw[mn[k]];
                         al = an > al ? an : al;
@@ -457,7 +473,7 @@ rhs_kernel(const RhsArgs a) {
                 al = an > al ? an : al;
             }
         }
-        dg_only = fabs(al) <= a.atol;
+        dg_only = fabs(al) <= kc.atol;
         alpha = (R)al;
     }
 
@@ -472,7 +488,7 @@ rhs_kernel(const RhsArgs a) {
             double sv[NV];
 #pragma unroll
             for (int v = 0; v < NV; ++v) sv[v] = 0.0;
-            if (EXT && a.src) source_at<DIM, NN, NV>(a, e, node, tnow, sv);
+            if (EXT && kc.src) source_at<DIM, NN, NV>(a, kc, e, node, tnow, sv);
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
                 R total = al[p][v];
@@ -511,8 +527,8 @@ rhs_kernel(const RhsArgs a) {
                     R f[NV];
                     node_flux<EQ, VF, TW, MEANS_ANY, R, L>(staged_node(base + i * s), nullptr,
                                                            staged_node(base + j * s), nullptr, d, P, f);
-                    const R fa = sc * (R)a.Ds[i * N + j];
-                    const R fb = sc * (R)a.Ds[j * N + i];
+                    const R fa = sc * (R)kc.Ds[i * N + j];
+                    const R fb = sc * (R)kc.Ds[j * N + i];
 #pragma unroll
                     for (int p = 0; p < N; ++p) {
                         const R w = p == i ? fa : (p == j ? fb : R(0));
@@ -536,32 +552,32 @@ rhs_kernel(const RhsArgs a) {
             um[v] = (R)um_next[v];
             up[v] = (R)up_next[v];
         }
-        if (EXT && a.bc) {
+        if (EXT && kc.bc) {
             // outflow sides: the inner face state on both sides, so that the
             // (consistent) surface flux is flux(u_inner)
             if (nb[2 * d] == -1) {
-                if ((a.outflow >> (2 * d)) & 1) {
+                if ((kc.outflow >> (2 * d)) & 1) {
 #pragma unroll
                     for (int v = 0; v < NV; ++v) um[v] = (R)U[soa(v, base, ec, slab, E32)];
-                } else if (a.bc == TRIXI_HIP_BC_SLIP_WALL) {
+                } else if (kc.bc == TRIXI_HIP_BC_SLIP_WALL) {
                     // slip wall: the inner state with its normal momentum reversed
 #pragma unroll
                     for (int v = 0; v < NV; ++v) um[v] = (R)U[soa(v, base, ec, slab, E32)];
                     um[1 + d] = -um[1 + d];
                 } else {
-                    boundary_state<DIM, NN, NV, R>(a, ec, base, tnow, um);
+                    boundary_state<DIM, NN, NV, R>(a, kc, ec, base, tnow, um);
                 }
             }
             if (nb[2 * d + 1] == -1) {
-                if ((a.outflow >> (2 * d + 1)) & 1) {
+                if ((kc.outflow >> (2 * d + 1)) & 1) {
 #pragma unroll
                     for (int v = 0; v < NV; ++v) up[v] = (R)U[soa(v, base + (N - 1) * s, ec, slab, E32)];
-                } else if (a.bc == TRIXI_HIP_BC_SLIP_WALL) {
+                } else if (kc.bc == TRIXI_HIP_BC_SLIP_WALL) {
 #pragma unroll
                     for (int v = 0; v < NV; ++v) up[v] = (R)U[soa(v, base + (N - 1) * s, ec, slab, E32)];
                     up[1 + d] = -up[1 + d];
                 } else {
-                    boundary_state<DIM, NN, NV, R>(a, ec, base + (N - 1) * s, tnow, up);
+                    boundary_state<DIM, NN, NV, R>(a, kc, ec, base + (N - 1) * s, tnow, up);
                 }
             }
         }
@@ -609,7 +625,7 @@ rhs_kernel(const RhsArgs a) {
                 const int r = threadIdx.x & 3;
                 float dh[N];
 #pragma unroll
-                for (int k = 0; k < N; ++k) dh[k] = (float)a.Dhat[r * N + k];
+                for (int k = 0; k < N; ++k) dh[k] = (float)kc.Dhat[r * N + k];
 #pragma unroll
                 for (int v = 0; v < NV; ++v) {
                     f32x4 c = {0.f, 0.f, 0.f, 0.f};
@@ -623,7 +639,7 @@ rhs_kernel(const RhsArgs a) {
                 for (int i = 0; i < N; ++i)
 #pragma unroll
                     for (int p = 0; p < N; ++p) {
-                        const R w = (R)a.Dhat[i * N + p];
+                        const R w = (R)kc.Dhat[i * N + p];
 #pragma unroll
                         for (int v = 0; v < NV; ++v) acl[i][v] += w * fl[p][v];
                     }
@@ -644,8 +660,8 @@ rhs_kernel(const RhsArgs a) {
                     for (int j = i + 1; j < N; ++j) {
                         R f[NV];
                         node_flux<EQ, VF, TW, MEANS_NEAR, R, L>(nd[i], nullptr, nd[j], nullptr, d, P, f);
-                        const R fa = sc * (R)a.Ds[i * N + j];
-                        const R fb = sc * (R)a.Ds[j * N + i];
+                        const R fa = sc * (R)kc.Ds[i * N + j];
+                        const R fb = sc * (R)kc.Ds[j * N + i];
 #pragma unroll
                         for (int v = 0; v < NV; ++v) {
                             acl[i][v] += fa * f[v];
@@ -669,7 +685,7 @@ rhs_kernel(const RhsArgs a) {
                     for (int j = 0; j < N; ++j) {
                         R f[NV];
                         EQ::template noncons<-1>(nd[i], nd[j], d, P, f);
-                        const R w = (R)a.Ds[i * N + j];
+                        const R w = (R)kc.Ds[i * N + j];
 #pragma unroll
                         for (int v = 0; v < NV; ++v) integral[v] += w * f[v];
                     }
@@ -690,8 +706,8 @@ rhs_kernel(const RhsArgs a) {
                         }
                     }
                     node_flux<EQ, FVF, TW, MEANS_ANY, R, L>(nd[p], ul, nd[p + 1], ur, d, P, F);
-                    const R wl = alpha * (R)a.invw[p];
-                    const R wr = alpha * (R)a.invw[p + 1];
+                    const R wl = alpha * (R)kc.invw[p];
+                    const R wr = alpha * (R)kc.invw[p + 1];
                     if constexpr (EQ::NONCONS) {
                         // subcell interface with nonconservative terms: the left
                         // node takes f + nc(u_l, u_r)/2, the right f + nc(u_r, u_l)/2
@@ -742,17 +758,17 @@ rhs_kernel(const RhsArgs a) {
             if constexpr (EXT) {
                 // mortar faces: the face node of this line is `line`
                 if (nb[2 * d] <= -2) {
-                    const double* mf = a.mflux + ((int64_t)(-2 - nb[2 * d]) * NL + line) * NV;
+                    const double* mf = kc.mflux + ((int64_t)(-2 - nb[2 * d]) * NL + line) * NV;
 #pragma unroll
                     for (int v = 0; v < NV; ++v) fm[v] = (TW ? R(2) : R(1)) * (R)mf[v];
                 }
                 if (nb[2 * d + 1] <= -2) {
-                    const double* mf = a.mflux + ((int64_t)(-2 - nb[2 * d + 1]) * NL + line) * NV;
+                    const double* mf = kc.mflux + ((int64_t)(-2 - nb[2 * d + 1]) * NL + line) * NV;
 #pragma unroll
                     for (int v = 0; v < NV; ++v) fp[v] = (TW ? R(2) : R(1)) * (R)mf[v];
                 }
             }
-            const R lm = (R)a.lhat_m, lp = (R)a.lhat_p;
+            const R lm = (R)kc.lhat_m, lp = (R)kc.lhat_p;
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
                 acl[0][v] = acl[0][v] - fm[v] * lm;
@@ -830,7 +846,7 @@ rhs_kernel(const RhsArgs a) {
             double sv[NV];
 #pragma unroll
             for (int v = 0; v < NV; ++v) sv[v] = 0.0;
-            if (EXT && a.src) source_at<DIM, NN, NV>(a, ee, n, tnow, sv);
+            if (EXT && kc.src) source_at<DIM, NN, NV>(a, kc, ee, n, tnow, sv);
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
                 const int64_t g = soa(v, n, ee, slab, E32);
@@ -890,7 +906,8 @@ __host__ __device__ constexpr int np_elems() {
 
 template <int DIM, int N, class EQ, int VOL, int VF, int SF, int FVF, typename R, bool RK, typename L, typename S>
 __global__ void __launch_bounds__((np_elems<DIM, N>() * cpow(N, DIM) * DIM))
-rhs_np_kernel(const RhsArgs a) {
+rhs_np_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
+    const RhsConst& kc = consts_of(consts);
     const S* __restrict__ U = static_cast<const S*>(a.u);
     S* __restrict__ DU = static_cast<S*>(a.du);
     S* __restrict__ K = static_cast<S*>(a.k);
@@ -930,7 +947,7 @@ rhs_np_kernel(const RhsArgs a) {
     const int64_t e = e0 + el;
     const bool valid = e < E;
     const int64_t ec = valid ? e : E - 1;
-    const PhysR<R> P = PhysR<R>::from(a.phys);
+    const PhysR<R> P = PhysR<R>::from(kc.phys);
     const bool last = d == DIM - 1;  // node pass and epilogue lanes
 
     // this node's position along direction d, and the interface state at the
@@ -969,14 +986,14 @@ rhs_np_kernel(const RhsArgs a) {
     bool dg_only = true;
     if constexpr (VOL == VI_HG) {
         double al = a.alpha_raw[ec];
-        if (a.smooth) {
+        if (kc.smooth) {
 #pragma unroll
             for (int f = 0; f < 2 * DIM; ++f) {
                 const double an = 0.5 * a.alpha_raw[a.nbr[(int64_t)f * E + ec]];
                 al = an > al ? an : al;
             }
         }
-        dg_only = fabs(al) <= a.atol;
+        dg_only = fabs(al) <= kc.atol;
         alpha = (R)al;
     }
 
@@ -1007,8 +1024,8 @@ rhs_np_kernel(const RhsArgs a) {
     for (int pp = 0; pp < N; ++pp) {
         if (pp != p) continue;
 #pragma unroll
-        for (int j = 0; j < N; ++j) dsr[j] = (R)a.Ds[pp * N + j];
-        invw_p = (R)a.invw[pp];
+        for (int j = 0; j < N; ++j) dsr[j] = (R)kc.Ds[pp * N + j];
+        invw_p = (R)kc.invw[pp];
     }
 
     // the direction's terms with the direction a compile-time constant (a
@@ -1113,7 +1130,7 @@ rhs_np_kernel(const RhsArgs a) {
     #pragma unroll
                 for (int v = 0; v < NV; ++v) fs[v] = fs[v] + R(0.5) * nc[v];
             }
-            const R lw = minus ? -(R)a.lhat_m : (R)a.lhat_p;
+            const R lw = minus ? -(R)kc.lhat_m : (R)kc.lhat_p;
     #pragma unroll
             for (int v = 0; v < NV; ++v) acl[v] = acl[v] + fs[v] * lw;
         }
@@ -1169,10 +1186,10 @@ rhs_np_kernel(const RhsArgs a) {
         // so the factors equal a separate indicator launch's bit for bit
         double* const buf = ind_buf;
         double* const e2 = ind_buf + M * NN;
-        const PhysR<double> P64 = PhysR<double>::from(a.phys);
-        const VinvRows<DIM, N> V = vinv_rows<DIM, N>(a.Vinv, node);
+        const PhysR<double> P64 = PhysR<double>::from(kc.phys);
+        const VinvRows<DIM, N> V = vinv_rows<DIM, N>(kc.Vinv, node);
         double m = 0.0;
-        if (last && valid) m = Euler<DIM>::indicator_variable(uo, P64, a.ind_var);
+        if (last && valid) m = Euler<DIM>::indicator_variable(uo, P64, kc.ind_var);
 #pragma unroll
         for (int dd = 0; dd < DIM; ++dd) {
             const int s2 = cpow(N, dd);
@@ -1192,8 +1209,8 @@ rhs_np_kernel(const RhsArgs a) {
         if (last && node == 0 && valid) {
             double total, clip1, clip2;
             modal_energies<DIM, N>(e2, el, total, clip1, clip2);
-            a.alpha_next[e] = hg_alpha(total, clip1, clip2, a.ind_threshold, a.ind_s, a.ind_alpha_min,
-                                       a.ind_alpha_max);
+            a.alpha_next[e] = hg_alpha(total, clip1, clip2, kc.ind_threshold, kc.ind_s, kc.ind_alpha_min,
+                                       kc.ind_alpha_max);
         }
     }
 }

@@ -739,6 +739,8 @@ struct trixi_hip_ctx {
     double* d_tmp = nullptr;  // RK stage states (two buffers of nvalues)
     int nblocks_red = 1024;
     RhsArgs args;
+    RhsConst consts;               // as on the device
+    RhsConst* d_consts = nullptr;
     LaunchFn rhs_fn = nullptr, rk_fn = nullptr;
     // adjoint
     VjpFn vjp_fn = nullptr;
@@ -812,7 +814,7 @@ static void free_ctx(trixi_hip_ctx* c) {
     if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
     if (c->graph) (void)hipGraphDestroy(c->graph);
     void* bufs[] = {c->d_nbr, c->d_invJ, c->d_x,     c->d_alpha_raw, c->d_alpha, c->d_time,
-                    c->d_partial, c->d_arrived, c->d_Vinv, c->d_Vdm,   c->d_wa,    c->d_w,
+                    c->d_partial, c->d_arrived, c->d_consts, c->d_Vinv, c->d_Vdm,   c->d_wa,    c->d_w,
                     c->d_tmp, c->d_stage, c->d_k, c->d_kbar, c->d_alphabar, c->d_winner, c->d_stage_alpha,
                     c->d_mids, c->d_mori, c->d_mls, c->d_mnb, c->d_mflux};
     for (void* p : bufs)
@@ -829,7 +831,7 @@ static int launch_indicator(trixi_hip_ctx* c, const void* u, hipStream_t s, bool
     double* const araw = out ? out : c->d_alpha_raw;
     const double threshold = 0.5 * pow(10.0, -1.8 * pow((double)c->N, 0.25));
     const double parameter_s = log((1.0 - 0.0001) / 0.0001);
-    const PhysParams& P = c->args.phys;
+    const PhysParams& P = c->consts.phys;
     if (c->N != 4 && c->N != 5) return fail(TRIXI_HIP_EUNSUPPORTED, "shock capturing is built for polydeg 3 and 4");
     const int var = c->cfg.equation == TRIXI_HIP_SHALLOW_WATER ? IND_WATERHEIGHT_PRESSURE : c->cfg.indicator_variable;
 #define TRIXI_HIP_IND_S(D, NQ, ST)                                                                             \
@@ -1165,6 +1167,7 @@ int trixi_hip_create(const trixi_hip_config* config, const trixi_hip_mesh* mesh,
     ALLOC(c->d_time, TIME_DOUBLES * sizeof(double));
     ALLOC(c->d_partial, (size_t)c->nblocks_red * 18 * sizeof(double));
     ALLOC(c->d_arrived, sizeof(unsigned));
+    ALLOC(c->d_consts, sizeof(RhsConst));
     c->h_result = take_result_slot();
     if (!c->h_result)
         return cleanup_fail(TRIXI_HIP_ENOMEM, "hipHostMalloc failed for the reduction results");
@@ -1218,47 +1221,51 @@ int trixi_hip_create(const trixi_hip_config* config, const trixi_hip_mesh* mesh,
 
     RhsArgs& a = c->args;
     memset(&a, 0, sizeof(a));
+    RhsConst& kc = c->consts;
+    memset(&kc, 0, sizeof(kc));
+    a.consts = c->d_consts;
+    a.host_consts = &c->consts;
     a.nbr = c->d_nbr;
     a.invJ = c->d_invJ;
     a.alpha_raw = c->d_alpha_raw;
     a.E = E;
-    a.phys.gamma = cfg.gamma;
-    a.phys.gm1 = cfg.gamma - 1.0;
-    a.phys.inv_gm1 = (cfg.gamma != 1.0) ? 1.0 / (cfg.gamma - 1.0) : 0.0;
-    a.phys.c_h = (cfg.equation == TRIXI_HIP_IDEAL_GLM_MHD && dim == 1) ? 0.0 : cfg.c_h;
+    kc.phys.gamma = cfg.gamma;
+    kc.phys.gm1 = cfg.gamma - 1.0;
+    kc.phys.inv_gm1 = (cfg.gamma != 1.0) ? 1.0 / (cfg.gamma - 1.0) : 0.0;
+    kc.phys.c_h = (cfg.equation == TRIXI_HIP_IDEAL_GLM_MHD && dim == 1) ? 0.0 : cfg.c_h;
     if (cfg.equation == TRIXI_HIP_HYPERBOLIC_DIFFUSION) {
-        a.phys.nu = cfg.nu;
-        a.phys.inv_Tr = cfg.nu / (cfg.Lr * cfg.Lr);  // T_r = Lr^2 / nu
+        kc.phys.nu = cfg.nu;
+        kc.phys.inv_Tr = cfg.nu / (cfg.Lr * cfg.Lr);  // T_r = Lr^2 / nu
     }
-    a.phys.grav = cfg.gravity;
+    kc.phys.grav = cfg.gravity;
     if (cfg.equation == TRIXI_HIP_COMPRESSIBLE_EULER_MULTICOMPONENT) {
         // c_v,k = R_k / (gamma_k - 1) (Trixi's cv), and c_v,k gamma_k
         for (int k = 0; k < cfg.ncomponents; ++k) {
-            a.phys.cv[k] = cfg.gas_constants[k] / (cfg.gammas[k] - 1.0);
-            a.phys.cvg[k] = a.phys.cv[k] * cfg.gammas[k];
+            kc.phys.cv[k] = cfg.gas_constants[k] / (cfg.gammas[k] - 1.0);
+            kc.phys.cvg[k] = kc.phys.cv[k] * cfg.gammas[k];
         }
     }
-    for (int d = 0; d < 3; ++d) a.phys.a[d] = cfg.advection_velocity[d];
-    a.bc_ic = ic_params(c, cfg.boundary_ic, cfg.boundary_seed);
+    for (int d = 0; d < 3; ++d) kc.phys.a[d] = cfg.advection_velocity[d];
+    kc.bc_ic = ic_params(c, cfg.boundary_ic, cfg.boundary_seed);
     for (int q = 0; q < N * N; ++q) {
-        a.Ds[q] = c->basis.Ds[q];
-        a.Dhat[q] = c->basis.Dhat[q];
+        kc.Ds[q] = c->basis.Ds[q];
+        kc.Dhat[q] = c->basis.Dhat[q];
     }
-    for (int q = 0; q < N; ++q) a.invw[q] = 1.0 / c->basis.w[q];
-    a.lhat_m = c->basis.lm[0];
-    a.lhat_p = c->basis.lp[N - 1];
+    for (int q = 0; q < N; ++q) kc.invw[q] = 1.0 / c->basis.w[q];
+    kc.lhat_m = c->basis.lm[0];
+    kc.lhat_p = c->basis.lp[N - 1];
     {
         const double eps = 2.220446049250313e-16;
-        a.atol = std::max(100 * eps, pow(eps, 0.75));
+        kc.atol = std::max(100 * eps, pow(eps, 0.75));
     }
-    a.smooth = cfg.alpha_smooth;
-    a.x = c->d_x;
-    a.bc = cfg.boundary_condition;
-    a.src = cfg.source_terms;
-    a.outflow = cfg.boundary_outflow_faces;
-    a.mflux = c->d_mflux;
-    a.mnb = c->d_mnb;
-    a.mK = K;
+    kc.smooth = cfg.alpha_smooth;
+    kc.x = c->d_x;
+    kc.bc = cfg.boundary_condition;
+    kc.src = cfg.source_terms;
+    kc.outflow = cfg.boundary_outflow_faces;
+    kc.mflux = c->d_mflux;
+    kc.mnb = c->d_mnb;
+    kc.mK = K;
     {
         MortarArgs& m = c->margs;
         memset(&m, 0, sizeof(m));
@@ -1268,7 +1275,7 @@ int trixi_hip_create(const trixi_hip_config* config, const trixi_hip_mesh* mesh,
         m.ls = c->d_mls;
         m.nmortars = NM;
         m.E = E;
-        m.phys = a.phys;
+        m.phys = kc.phys;
         if (NM > 0) mortar_operators(c->basis, N, m.F, m.R);
     }
     a.nxcd = 1;
@@ -1302,18 +1309,20 @@ int trixi_hip_create(const trixi_hip_config* config, const trixi_hip_mesh* mesh,
         // for the fused RK stages of the node-parallel form, which write the
         // next stage's raw blending factors; TRIXI_HIP_FUSE_INDICATOR=0 keeps
         // a separate indicator launch per stage
-        a.Vinv = c->d_Vinv;
-        a.ind_threshold = 0.5 * pow(10.0, -1.8 * pow((double)N, 0.25));
-        a.ind_s = log((1.0 - 0.0001) / 0.0001);
-        a.ind_alpha_min = cfg.alpha_min;
-        a.ind_alpha_max = cfg.alpha_max;
-        a.ind_var = cfg.indicator_variable;
+        kc.Vinv = c->d_Vinv;
+        kc.ind_threshold = 0.5 * pow(10.0, -1.8 * pow((double)N, 0.25));
+        kc.ind_s = log((1.0 - 0.0001) / 0.0001);
+        kc.ind_alpha_min = cfg.alpha_min;
+        kc.ind_alpha_max = cfg.alpha_max;
+        kc.ind_var = cfg.indicator_variable;
         const char* fenv = getenv("TRIXI_HIP_FUSE_INDICATOR");
         c->fuse_ind = a.np && cfg.volume_integral == TRIXI_HIP_VOLUME_SHOCK_CAPTURING_HG &&
                       cfg.equation == TRIXI_HIP_COMPRESSIBLE_EULER && (N == 4 || N == 5) &&
                       !(fenv && atoi(fenv) == 0);
     }
     {
+        if (hipMemcpy(c->d_consts, &c->consts, sizeof(RhsConst), hipMemcpyHostToDevice) != hipSuccess)
+            return cleanup_fail(TRIXI_HIP_EDEVICE, "host to device copy failed in create");
         // look up this device's static scratch once, at set-up, with the
         // device current (used by the *_noalloc entry points)
         double* sp = nullptr;
@@ -1400,7 +1409,7 @@ static IcParams ic_params(const trixi_hip_ctx* c, int ic, uint64_t seed) {
     q.nv = c->nv;
     q.ic = ic;
     q.gamma = c->cfg.gamma;
-    q.inv_gm1 = c->args.phys.inv_gm1;
+    q.inv_gm1 = c->consts.phys.inv_gm1;
     q.c_h = c->cfg.c_h;
     for (int d = 0; d < 3; ++d) q.a[d] = c->cfg.advection_velocity[d];
     q.length = c->cfg.ic_length;
@@ -1408,8 +1417,8 @@ static IcParams ic_params(const trixi_hip_ctx* c, int ic, uint64_t seed) {
     q.nc = c->cfg.equation == TRIXI_HIP_COMPRESSIBLE_EULER_MULTICOMPONENT ? c->cfg.ncomponents : 0;
     q.grav = c->cfg.gravity;
     for (int k = 0; k < MAXC; ++k) {
-        q.cv[k] = c->args.phys.cv[k];
-        q.cvg[k] = c->args.phys.cvg[k];
+        q.cv[k] = c->consts.phys.cv[k];
+        q.cvg[k] = c->consts.phys.cvg[k];
     }
     return q;
 }
@@ -1572,7 +1581,7 @@ static int reduction_blocks(const trixi_hip_ctx* c) {
 extern "C++" template <typename S>
 static int launch_max_speed(trixi_hip_ctx* ctx, const S* u, hipStream_t s, int blocks, double* partial,
                             double* result, unsigned* arrived, const StepControl& step = StepControl{}) {
-    const PhysParams& P = ctx->args.phys;
+    const PhysParams& P = ctx->consts.phys;
     const int eq = ctx->cfg.equation, dim = ctx->dim;
 #define MS(EQT, D)                                                                                                 \
     hipLaunchKernelGGL((max_speed_kernel<EQT, D, S>), dim3(blocks), dim3(RED_THREADS), 0, s, u, ctx->d_invJ, partial, \
@@ -1842,14 +1851,14 @@ static VjpArgs vjp_args(const trixi_hip_ctx* c) {
     v.nbr = c->d_nbr;
     v.invJ = c->d_invJ;
     v.E = c->E;
-    v.phys = c->args.phys;
+    v.phys = c->consts.phys;
     for (int q = 0; q < MAXN * MAXN; ++q) {
-        v.Ds[q] = c->args.Ds[q];
-        v.Dhat[q] = c->args.Dhat[q];
+        v.Ds[q] = c->consts.Ds[q];
+        v.Dhat[q] = c->consts.Dhat[q];
     }
-    for (int q = 0; q < MAXN; ++q) v.invw[q] = c->args.invw[q];
-    v.lhat_m = c->args.lhat_m;
-    v.lhat_p = c->args.lhat_p;
+    for (int q = 0; q < MAXN; ++q) v.invw[q] = c->consts.invw[q];
+    v.lhat_m = c->consts.lhat_m;
+    v.lhat_p = c->consts.lhat_p;
     v.nxcd = c->args.nxcd;
     // the direction-group form below two waves per SIMD of the one-group
     // form (as the rhs kernel's node-parallel form); 0 turns it off
@@ -1858,11 +1867,11 @@ static VjpArgs vjp_args(const trixi_hip_ctx* c) {
     v.alpha_raw = c->d_alpha_raw;
     v.alphabar = c->d_alphabar;
     v.winner = c->d_winner;
-    v.atol = c->args.atol;
-    v.smooth = c->args.smooth;
+    v.atol = c->consts.atol;
+    v.smooth = c->consts.smooth;
     v.x = c->d_x;
-    v.bc_ic = c->args.bc_ic;
-    v.bc = c->args.bc;
+    v.bc_ic = c->consts.bc_ic;
+    v.bc = c->consts.bc;
     return v;
 }
 
@@ -1919,7 +1928,7 @@ static int enqueue_vjp(trixi_hip_ctx* c, const VjpArgs& v, hipStream_t s, bool a
         const int threads = 64;
         const double threshold = 0.5 * pow(10.0, -1.8 * pow((double)c->N, 0.25));
         const double parameter_s = log((1.0 - 0.0001) / 0.0001);
-        const PhysParams& P = c->args.phys;
+        const PhysParams& P = c->consts.phys;
 #define TRIXI_HIP_IND_VJP(D)                                                                                    \
     hipLaunchKernelGGL((indicator_vjp_kernel<D, 4>), dim3(blocks), dim3(threads), 0, s, v.u, v.ubar,            \
                        (const double*)c->d_alphabar, (const int32_t*)c->d_winner, (const int32_t*)c->d_nbr,    \
@@ -2061,7 +2070,7 @@ int trixi_hip_check_state(trixi_hip_ctx* ctx, const double* u, int32_t* flags, i
     const int threads = 256;
     const int blocks = (int)std::min<int64_t>((ctx->E + threads - 1) / threads, ctx->nblocks_red);
     hipLaunchKernelGGL(check_state_kernel, dim3(blocks), dim3(threads), 0, s, u, flags, ctx->d_partial,
-                       ctx->h_result, ctx->d_arrived, ctx->cfg.equation, ctx->dim, ctx->nv, ctx->nn, ctx->E, ctx->args.phys);
+                       ctx->h_result, ctx->d_arrived, ctx->cfg.equation, ctx->dim, ctx->nv, ctx->nn, ctx->E, ctx->consts.phys);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s));
     *nbad = (int64_t)ctx->h_result[0];
