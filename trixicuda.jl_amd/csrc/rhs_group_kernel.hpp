@@ -428,7 +428,13 @@ __global__ void __launch_bounds__((group_threads<DIM, N, M>()), WAVES) rhs_group
     int tid2 = tid;
     asm volatile("" : "+v"(tid2));
 
-    // u and k of the register update, requested before the sums meet
+    // the element's scale and dt, and u and k of the register update, requested
+    // before the sums meet (a lane's nodes of the final pass are of one element:
+    // NT is a multiple of M)
+    static_assert(NT % M == 0, "a lane's nodes belong to one element");
+    const double invj = a.invJ[e0 + tid2 % M < E ? e0 + tid2 % M : E - 1];
+    double t_dt = 0.0;
+    if (RK) t_dt = a.time[1];
     double uu[RK ? NIT : 1][NV], kk[RK ? NIT : 1][NV];
     const double* __restrict__ K = static_cast<const double*>(a.k);
     if constexpr (RK) {
@@ -494,13 +500,11 @@ __global__ void __launch_bounds__((group_threads<DIM, N, M>()), WAVES) rhs_group
                 for (int v = 0; v < NV; ++v) t[v] += fcs[(((2 * d + side) * NL + ln) * NV + v) * M + c];
             }
         }
-        const double fac = (TW ? -0.5 : -1.0) * a.invJ[e];
+        const double fac = (TW ? -0.5 : -1.0) * invj;
         double sv[NV];
 #pragma unroll
         for (int v = 0; v < NV; ++v) sv[v] = 0.0;
         if (EXT && kc.src) source_at<DIM, NN, NV>(a, kc, e, n, tnow, sv);
-        double t_dt = 0.0;
-        if (RK) t_dt = a.time[1];
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             const int64_t g = soa(v, n, e, slab, E32);

@@ -387,6 +387,11 @@ rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
     // order, so the node pass then waits for its own data only
     if constexpr (EARLY) __builtin_amdgcn_sched_barrier(0);
 
+    // the scale of the element's sums (a lane's nodes of the final pass belong to
+    // its element too: NT is a multiple of M) and dt, ahead of the fluxes
+    const double invj = a.invJ[ec];
+    double t_dt = 0.0;
+    if (RK) t_dt = a.time[1];
     double tnow = 0.0;
     if constexpr (EXT) tnow = RK ? a.time[0] : a.t_host;
     double um_next[NV], up_next[NV];
@@ -479,9 +484,7 @@ rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
 
     // last direction, sequential or not: -1/J (+ sources), then du or the RK update
     auto line_epilogue = [&](R (&al)[N][NV], int base, int s) {
-        const double fac = (TW ? -0.5 : -1.0) * a.invJ[e];
-        double t_dt = 0.0;
-        if (RK) t_dt = a.time[1];
+        const double fac = (TW ? -0.5 : -1.0) * invj;
 #pragma unroll
         for (int p = 0; p < N; ++p) {
             const int node = base + p * s;
@@ -833,7 +836,7 @@ rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
         // k = a_s k + dt du, u_out = u + b_s k over the node pass's pairs;
         // the accumulator holds every direction (same summation order as the
         // line-wise path)
-        const double t_dt = a.time[1];
+        static_assert(NT % M == 0, "a lane's nodes belong to its element");
 #pragma unroll
         for (int it = 0; it < NIT; ++it) {
             const int q = tid + it * NT;
@@ -842,7 +845,7 @@ rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
             const int n = q / M;
             const int64_t ee = e0 + c;
             if (ee >= E) continue;
-            const double fac = (TW ? -0.5 : -1.0) * a.invJ[ee];
+            const double fac = (TW ? -0.5 : -1.0) * invj;
             double sv[NV];
 #pragma unroll
             for (int v = 0; v < NV; ++v) sv[v] = 0.0;
@@ -957,6 +960,26 @@ rhs_np_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
     const int base = node - p * s;
     const bool face = p == 0 || p == N - 1;
     R ub[NV];
+    // (everything this kernel reads from memory is requested here, ahead of the
+    // node pass: on the small meshes it runs, a load behind a barrier or in the
+    // epilogue is latency that nothing hides)
+    int32_t nbf[2 * DIM];
+    if constexpr (VOL == VI_HG) {
+#pragma unroll
+        for (int f = 0; f < 2 * DIM; ++f) nbf[f] = a.nbr[(int64_t)f * E + ec];
+    }
+    S us[NV], ks[RK ? NV : 1];
+    if (last) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const int64_t g = soa(v, node, ec, slab, E32);
+            us[v] = U[g];
+            if constexpr (RK) ks[v] = a.rk_first ? S(0) : K[g];
+        }
+    }
+    const double invj = a.invJ[ec];
+    double t_dt = 0.0;
+    if (RK) t_dt = a.time[1];
     if (face) {
         const int32_t nbe = a.nbr[(int64_t)(2 * d + (p == 0 ? 0 : 1)) * E + ec];
         const int nn_face = p == 0 ? node + (N - 1) * s : node - (N - 1) * s;
@@ -964,12 +987,19 @@ rhs_np_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
         for (int v = 0; v < NV; ++v) ub[v] = (R)U[soa(v, nn_face, nbe, slab, E32)];
     }
 
+    double araw[2 * DIM + 1];
+    if constexpr (VOL == VI_HG) {
+        araw[2 * DIM] = a.alpha_raw[ec];
+#pragma unroll
+        for (int f = 0; f < 2 * DIM; ++f) araw[f] = kc.smooth ? a.alpha_raw[nbf[f]] : 0.0;
+    }
+
     if (RK && a.done != nullptr && *a.done != 0.0) return;  // uniform
 
     if (last) {
         R uc[NV];
 #pragma unroll
-        for (int v = 0; v < NV; ++v) uc[v] = (R)U[soa(v, node, ec, slab, E32)];
+        for (int v = 0; v < NV; ++v) uc[v] = (R)us[v];
         const Node nd = EQ::template node<R, NODE_LOGS, L>(uc, P);
         R f[NRF];
         EQ::to_rec(nd, f);
@@ -985,11 +1015,11 @@ rhs_np_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
     R alpha = R(0);
     bool dg_only = true;
     if constexpr (VOL == VI_HG) {
-        double al = a.alpha_raw[ec];
+        double al = araw[2 * DIM];
         if (kc.smooth) {
 #pragma unroll
             for (int f = 0; f < 2 * DIM; ++f) {
-                const double an = 0.5 * a.alpha_raw[a.nbr[(int64_t)f * E + ec]];
+                const double an = 0.5 * araw[f];
                 al = an > al ? an : al;
             }
         }
@@ -1153,9 +1183,7 @@ rhs_np_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
     // (no early exit: the fused indicator below synchronises the workgroup)
     double uo[FUSE_IND ? NV : 1];
     if (last && valid) {
-        const double fac = (TW ? -0.5 : -1.0) * a.invJ[e];
-        double t_dt = 0.0;
-        if (RK) t_dt = a.time[1];
+        const double fac = (TW ? -0.5 : -1.0) * invj;
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             R total = acl[v];
@@ -1170,10 +1198,9 @@ rhs_np_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
             if constexpr (!RK) {
                 DU[g] = (S)val;
             } else {
-                // u and k again (cache resident on the small meshes this form runs)
-                const S kk = (S)(a.rk_first ? t_dt * val : a.rk_a * (double)K[g] + t_dt * val);
+                const S kk = (S)(a.rk_first ? t_dt * val : a.rk_a * (double)ks[v] + t_dt * val);
                 K[g] = kk;
-                const S un = (S)((double)U[g] + a.rk_b * (double)kk);
+                const S un = (S)((double)us[v] + a.rk_b * (double)kk);
                 UO[g] = un;
                 if constexpr (FUSE_IND) uo[v] = (double)un;
             }
