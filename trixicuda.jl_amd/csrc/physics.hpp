@@ -584,8 +584,8 @@ struct Euler {
     }
     // whether every pair of these nodes satisfies MEANS_NEAR: rho, and rho / p
     // through the staged sound speed (rho / p = gamma / c^2)
-    template <int N, typename L>
-    __device__ static bool near_line(const Node<double, L>* n) {
+    template <int N, class ND>
+    __device__ static bool near_line(const ND* n) {
         double r0 = n[0].rho, r1 = r0, c0 = n[0].c, c1 = c0, p0 = n[0].p;
 #pragma unroll
         for (int i = 1; i < N; ++i) {

@@ -66,6 +66,73 @@ __device__ __forceinline__ void inv_ln_mean_grad(R x, R y, double lx, double ly,
     }
 }
 
+// ln_mean(x1, y1) and inv_ln_mean(x2, y2) with their partial derivatives, FP64,
+// without logarithms, in the ranges of the forward log_free_means:
+//   L = s Q(z^2):    L_x = Q - 4 y z Q' / s,            L_y = Q + 4 x z Q' / s
+//   I = P(z^2) / s:  I_x = -(P + 4 y z P' / s) / s^2,   I_y = (4 x z P' / s - P) / s^2
+// Q and P of degree 7 are the integrals of minimax polynomials of their
+// derivatives (relative errors 1.1e-16 and 6.1e-16; of the values below 1e-18),
+// value and derivative from one Horner scheme, so that both share the
+// coefficients: with polynomials of their own the 28 of them no longer fitted
+// the scalar registers.  Beyond |z| < 0.15 the closed forms with log(y / x).
+template <int MEANS>
+__device__ __forceinline__ void log_free_mean_grads(double x1, double y1, double x2, double y2, double& L, double& Lx,
+                                                    double& Ly, double& I, double& Ix, double& Iy) {
+    const double s1 = x1 + y1, d1 = y1 - x1;
+    const double s2 = x2 + y2, d2 = y2 - x2;
+    const double r = rrcp(s1 * s2);
+    const double r1 = r * s2, r2 = r * s1;
+    const double z1 = d1 * r1, z2 = d2 * r2;
+    const double q1 = z1 * z1, q2 = z2 * z2;
+    double Q = fastlog_const<true>(-0.007279622637948864), Qd = Q;
+    const double cq[6] = {-0.008374415772938017, -0.010898761130780577, -0.015096998212600984,
+                          -0.023280423298230768, -0.0444444444444068,   -0.16666666666666669};
+    double Pq = fastlog_const<true>(0.14444932391800686), Pd = Pq;
+    const double cp[6] = {0.15343866096875258, 0.18182573827691864, 0.2222221475487719,
+                          0.28571428608841193, 0.3999999999992102,  0.6666666666666671};
+    Q = fma(q1, Q, fastlog_const<true>(cq[0]));
+    Pq = fma(q2, Pq, fastlog_const<true>(cp[0]));
+#pragma unroll
+    for (int k = 1; k < 6; ++k) {
+        Qd = fma(q1, Qd, Q);
+        Q = fma(q1, Q, fastlog_const<true>(cq[k]));
+        Pd = fma(q2, Pd, Pq);
+        Pq = fma(q2, Pq, fastlog_const<true>(cp[k]));
+    }
+    Qd = fma(q1, Qd, Q);
+    Q = fma(q1, Q, 0.5);
+    Pd = fma(q2, Pd, Pq);
+    Pq = fma(q2, Pq, 2.0);
+    const double t1 = 4.0 * z1 * r1 * Qd;
+    L = s1 * Q;
+    Lx = fma(-y1, t1, Q);
+    Ly = fma(x1, t1, Q);
+    const double rr = r2 * r2;
+    const double t2 = 4.0 * z2 * r2 * Pd;
+    I = Pq * r2;
+    Ix = -rr * fma(y2, t2, Pq);
+    Iy = rr * fma(x2, t2, -Pq);
+    if constexpr (MEANS == MEANS_ANY) {
+        // (false for nonpositive sums and NaN, which then go through the logarithm)
+        const bool near1 = fabs(d1) < 0.15 * s1, near2 = fabs(d2) < 0.15 * s2;
+        if (__builtin_amdgcn_ballot_w64(!(near1 && near2)) != 0) {
+            const double nan = __builtin_nan("");
+            if (!near1) {
+                const double k = rdiv(1.0, x1 > 0.0 ? fast_log<true>(rdiv(y1, x1)) : nan);
+                L = d1 * k;
+                Lx = (L * rrcp(x1) - 1.0) * k;
+                Ly = (1.0 - L * rrcp(y1)) * k;
+            }
+            if (!near2) {
+                const double k = rdiv(1.0, d2);
+                I = (x2 > 0.0 ? fast_log<true>(rdiv(y2, x2)) : nan) * k;
+                Ix = (I - rrcp(x2)) * k;
+                Iy = (rrcp(y2) - I) * k;
+            }
+        }
+    }
+}
+
 // ===========================================================================
 // Linear scalar advection.
 // ===========================================================================
@@ -145,7 +212,7 @@ struct EulerVjp {
         R rho, v[DIM], p;
     };
 
-    template <typename R>
+    template <typename R, bool LOGS = true>
     __device__ static Node<R> node(const R* u, const PhysR<R>& P) {
         Node<R> n;
         n.rho = u[0];
@@ -159,8 +226,22 @@ struct EulerVjp {
         n.p = P.gm1 * (u[DIM + 1] - R(0.5) * ke);
         n.ip = rrcp(n.p);
         n.c = rsqrt_(P.gamma * n.p * n.irho);
-        n.lrho = node_log((double)n.rho);
-        n.lp = node_log((double)n.p);
+        n.lrho = LOGS ? node_log((double)n.rho) : 0.0;
+        n.lp = LOGS ? node_log((double)n.p) : 0.0;
+        return n;
+    }
+    // a record of (rho, v, p, c) without logarithms
+    template <typename R>
+    __device__ static Node<R> from_short_rec(const R* f) {
+        Node<R> n;
+        n.rho = f[0];
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) n.v[d] = f[1 + d];
+        n.p = f[DIM + 1];
+        n.c = f[DIM + 2];
+        n.irho = rrcp(n.rho);
+        n.ip = rrcp(n.p);
+        n.lrho = n.lp = 0.0;
         return n;
     }
     template <typename R>
@@ -303,15 +384,107 @@ struct EulerVjp {
         b.rho -= h * n.irho;
     }
 
-    template <int KIND, typename R>
+    // flux_ranocha with the means and derivatives of log_free_mean_grads (L of
+    // the densities, I of rho_l p_r and rho_r p_l); h is half the flux's
+    // cotangent, so that the averages' halves cancel.
+    __device__ static void ranocha_vjp(const Node<double>& l, const Node<double>& r, int o, const double* h,
+                                       Bar<double>& bl, Bar<double>& br, const PhysR<double>& P, double L, double Lx,
+                                       double Ly, double I, double Ix, double Iy) {
+        const double hE = h[DIM + 1], pp = l.p * r.p;
+        double f1b = 2.0 * h[0], S = 0.0;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+            f1b = fma(h[1 + d], l.v[d] + r.v[d], f1b);
+            S = fma(l.v[d], r.v[d], S);
+        }
+        f1b = fma(hE, fma(2.0 * P.inv_gm1 * pp, I, S), f1b);
+        const double V = l.v[o] + r.v[o];
+        const double f1 = L * (0.5 * V), q = 0.5 * f1b, a = hE * f1;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+            if (d == o) {
+                const double t = fma(q, L, h[1 + d] * f1);
+                bl.v[d] += t;
+                br.v[d] += t;
+                bl.v[d] = fma(hE, r.p, bl.v[d]);
+                br.v[d] = fma(hE, l.p, br.v[d]);
+            } else {
+                bl.v[d] = fma(h[1 + d], f1, bl.v[d]);
+                br.v[d] = fma(h[1 + d], f1, br.v[d]);
+            }
+            bl.v[d] = fma(a, r.v[d], bl.v[d]);
+            br.v[d] = fma(a, l.v[d], br.v[d]);
+        }
+        const double Bb = 2.0 * P.inv_gm1 * a, w = Bb * I, Ib = Bb * pp;
+        const double X = Ib * Ix, Y = Ib * Iy, m = q * V;
+        bl.p = fma(Y, r.rho, fma(w, r.p, fma(hE, r.v[o], bl.p + h[1 + o])));
+        br.p = fma(X, l.rho, fma(w, l.p, fma(hE, l.v[o], br.p + h[1 + o])));
+        bl.rho = fma(X, r.p, fma(m, Lx, bl.rho));
+        br.rho = fma(Y, l.p, fma(m, Ly, br.rho));
+    }
+
+    // The cotangent of one side of an interface flux, `own` (on the right of
+    // `nbr`, whose conservative state is un, or on its left), FP64 without node
+    // logarithms: two_point_vjp with the other side's left out.
+    template <int KIND, bool RIGHT>
+    __device__ static void own_side_vjp(const Node<double>& own, const Node<double>& nbr, const double* un, int o,
+                                        const double* g, Bar<double>& b, const PhysR<double>& P) {
+        if constexpr (KIND == FLUX_LLF || KIND == FLUX_LLF_NAIVE) {
+            // f = (f_l + f_r)/2 - lam/2 (u_r - u_l); the physical flux is u v_o
+            // and the pressure terms, so that v_o and lam scale the same vector
+            const double ao = dabs(own.v[o]), an = dabs(nbr.v[o]);
+            double lam;
+            bool sel_v, sel_c;  // lam's speeds are this side's (the left's if equal)
+            if (KIND == FLUX_LLF_NAIVE) {
+                sel_v = RIGHT ? ao > an : !(an > ao);
+                sel_c = RIGHT ? own.c > nbr.c : !(nbr.c > own.c);
+                lam = (sel_v ? ao : an) + (sel_c ? own.c : nbr.c);
+            } else {
+                sel_v = sel_c = RIGHT ? ao + own.c > an + nbr.c : !(an + nbr.c > ao + own.c);
+                lam = sel_v ? ao + own.c : an + nbr.c;
+            }
+            const double s = RIGHT ? own.v[o] - lam : own.v[o] + lam;
+            double c[NV], hu = 0.0, jump = 0.0;
+#pragma unroll
+            for (int q = 0; q < NV; ++q) {
+                const double h = 0.5 * g[q];
+                c[q] = h * s;
+                const double uo = cons(own, q, P);
+                hu = fma(h, uo, hu);
+                jump = fma(h, un[q] - uo, jump);
+            }
+            add_cons_bar(own, c, b, P);
+            const double hE = 0.5 * g[DIM + 1];
+            b.p += fma(hE, own.v[o], 0.5 * g[1 + o]);
+            const double lb = RIGHT ? jump : -jump;
+            const double lv = sel_v ? lb : 0.0, lc = sel_c ? lb : 0.0;
+            b.v[o] += fma(hE, own.p, hu) + (own.v[o] >= 0.0 ? lv : -lv);
+            sound_vjp(own, lc, b);
+        } else {
+            Bar<double> other;
+            zero(other);
+            if (RIGHT)
+                two_point_vjp<KIND, MEANS_ANY>(nbr, own, o, g, other, b, P);
+            else
+                two_point_vjp<KIND, MEANS_ANY>(own, nbr, o, g, b, other, P);
+        }
+    }
+
+    // MEANS: which logarithmic means; 0 takes the nodes' logarithms, others
+    // (FP64) log_free_mean_grads
+    template <int KIND, int MEANS = 0, typename R>
     __device__ static void two_point_vjp(const Node<R>& l, const Node<R>& r, int o, const R* g, Bar<R>& bl,
                                          Bar<R>& br, const PhysR<R>& P) {
         if (KIND == FLUX_RANOCHA) {
             R rho_mean, dLx, dLy;
-            ln_mean_grad<R>(l.rho, r.rho, l.lrho, r.lrho, l.irho, r.irho, rho_mean, dLx, dLy);
             const R X = l.rho * r.p, Y = r.rho * l.p;
             R I, dIx, dIy;
-            inv_ln_mean_grad<R>(X, Y, l.lrho + r.lp, r.lrho + l.lp, l.irho * r.ip, r.irho * l.ip, I, dIx, dIy);
+            if constexpr (MEANS != 0) {
+                log_free_mean_grads<MEANS>(l.rho, r.rho, X, Y, rho_mean, dLx, dLy, I, dIx, dIy);
+            } else {
+                ln_mean_grad<R>(l.rho, r.rho, l.lrho, r.lrho, l.irho, r.irho, rho_mean, dLx, dLy);
+                inv_ln_mean_grad<R>(X, Y, l.lrho + r.lp, r.lrho + l.lp, l.irho * r.ip, r.irho * l.ip, I, dIx, dIy);
+            }
             const R B = l.p * r.p * I;
             R va[DIM], vs = R(0);
 #pragma unroll

@@ -3,7 +3,7 @@
 
 #include "launch_rhs.hpp"
 #include "mortar_kernel.hpp"
-#include "vjp_kernel.hpp"
+#include "vjp_group_kernel.hpp"
 
 namespace trixi_hip {
 

@@ -73,8 +73,9 @@ struct VjpArgs {
 // nine-variable MHD adjoint: whole waves per direction group; gfx950 gives a
 // workgroup up to 160 KiB of LDS).  The one-group form (large meshes) takes
 // up to 128 KiB: 3D Euler at level 5 with 8-element tiles, VJP 165 -> 159 us
-// (the direction-group forms of the small meshes measured slower with wider
-// tiles).
+// (flux differencing, before it had the lane-group form of
+// vjp_group_kernel.hpp; the direction-group forms of the small meshes measured
+// slower with wider tiles).
 template <int DIM, int N, int NV, int NRF, int G, int GA>
 __host__ __device__ constexpr int vjp_width() {
     constexpr int NL = cpow(N, DIM - 1), NN = cpow(N, DIM);
@@ -621,29 +622,6 @@ vjp_kernel(const VjpArgs a) {
             if (a.kbar_out != nullptr) a.kbar_out[g] = a.kbar_a * a.vbar[g] + a.kbar_b * ubn;
         }
     }
-}
-
-// M: elements per workgroup of the one-group form; MG: of the
-// direction-group form, used for meshes whose one-group form would launch
-// fewer lanes than a.pd_lanes (on 2D and 3D meshes).
-template <int DIM, int N, class EQ, int VOL, int VF, int SF, int FVF, typename R, int M, bool EXT = false,
-          int MG = M>
-hipError_t launch_vjp(const VjpArgs& a, hipStream_t stream) {
-    constexpr int NL = cpow(N, DIM - 1);
-    if constexpr (DIM > 1) {
-        if (a.E * NL < a.pd_lanes) {
-            int64_t blocks = (a.E + MG - 1) / MG;
-            if (a.nxcd > 1) blocks = (blocks + a.nxcd - 1) / a.nxcd * a.nxcd;
-            hipLaunchKernelGGL((vjp_kernel<DIM, N, EQ, VOL, VF, SF, FVF, R, MG, EXT, DIM>), dim3((unsigned)blocks),
-                               dim3(MG * NL * vjp_groups<DIM, N, VOL, EQ::NV, EQ::NRF, DIM>()), 0, stream, a);
-            return hipGetLastError();
-        }
-    }
-    int64_t blocks = (a.E + M - 1) / M;
-    if (a.nxcd > 1) blocks = (blocks + a.nxcd - 1) / a.nxcd * a.nxcd;
-    hipLaunchKernelGGL((vjp_kernel<DIM, N, EQ, VOL, VF, SF, FVF, R, M, EXT, 1>), dim3((unsigned)blocks), dim3(M * NL),
-                       0, stream, a);
-    return hipGetLastError();
 }
 
 }  // namespace trixi_hip
