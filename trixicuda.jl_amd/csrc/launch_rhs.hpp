@@ -65,8 +65,14 @@ hipError_t launch_rhs(const RhsArgs& a, hipStream_t stream) {
     if (a.alpha_next != nullptr) return hipErrorInvalidValue;
     if constexpr (group_eligible<DIM, N, EQ, VOL, R>()) {
         constexpr int ME = group_elems<DIM, N, EQ::NV, EQ::NRF>();
-        constexpr int MG = EXT && (ME / 2 * cpow(N, DIM - 1)) % 64 == 0 ? ME / 2 : ME;
-        constexpr int W = EQ::NV > 5 || EXT ? 2 : (DIM == 3 ? 4 : TRIXI_HIP_GROUP_WAVES2D);
+        // Half the elements and two waves per SIMD (256 registers) where four
+        // waves spill: boundary and mortar faces, and shock capturing in 3D,
+        // whose blended lines hold 60 registers too many (rhs! at 32768
+        // elements 219 -> 180 us, three CFL steps 4360 -> 3320; with three
+        // waves the same).
+        constexpr bool HALF = EXT || (VOL == VI_HG && DIM == 3);
+        constexpr int MG = HALF && (ME / 2 * cpow(N, DIM - 1)) % 64 == 0 ? ME / 2 : ME;
+        constexpr int W = EQ::NV > 5 || HALF ? 2 : (DIM == 3 ? 4 : TRIXI_HIP_GROUP_WAVES2D);
         hipLaunchKernelGGL((rhs_group_kernel<DIM, N, EQ, VOL, VF, SF, FVF, MG, RK, EXT, W>), grid(MG),
                            dim3(group_threads<DIM, N, MG>()), 0, stream, a, a.consts);
     } else {
