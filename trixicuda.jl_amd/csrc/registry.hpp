@@ -55,8 +55,8 @@ struct VjpRegistrar {
 // with FP32 arithmetic and up to five variables, whose wider tiles (3D Euler: 16 elements, whole
 // 128-byte rows of an FP64 state) measured faster despite two waves per SIMD
 // instead of 2.5: 3D Euler level 5, mixed rhs! 57.2 -> 54.9 us, FP32-state
-// rhs! 45.0 -> 40.4 us, RK steps -11 % and -8 % (the FP64 kernel at 8
-// elements: 80 -> 101 us).
+// rhs! 45.0 -> 40.4 us, RK steps -11 % and -8 % (FP64 in this form at 8
+// elements: 80 -> 101 us; rhs_group_kernel has its own widths, group_elems).
 #ifndef TRIXI_HIP_LDS_BUDGET_KIB
 #define TRIXI_HIP_LDS_BUDGET_KIB 40
 #endif

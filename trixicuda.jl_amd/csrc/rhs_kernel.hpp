@@ -239,12 +239,14 @@ __device__ __forceinline__ int line_base(int line, int d) {
 // its own M * N^(d-1) lanes (whole waves), otherwise one group runs the
 // directions one after the other.  Parallel directions triple the waves per
 // element, which pays where LDS or registers limit the occupancy of the
-// sequential form: the FP64 rhs! (3D Euler flux differencing at level 5:
-// 93.8 -> 89.5 us) and the FP64 fused RK stage (fewer registers than the
-// sequential form's 256).  In FP32 arithmetic (63.4 -> 76.8 us) the
-// sequential form stays, with one copy of each direction's code live at a
-// time, and so it does for the nine-variable MHD system, whose parallel form
-// spills (3D GLM-MHD at level 4: 28.6 -> 45.5 us).
+// sequential form: FP64 rhs! and RK stages.  (Measured with 3D Euler flux
+// differencing at level 5, 93.8 -> 89.5 us, before that configuration had
+// rhs_group_kernel; what runs this form now are the FP64 weak forms, the
+// equations without a lane-group form and node counts that do not fill waves.)
+// In FP32 arithmetic (63.4 -> 76.8 us) the sequential form stays, with one
+// copy of each direction's code live at a time, and so it does for systems of
+// more than five variables, whose parallel form spills (3D GLM-MHD at level 4:
+// 28.6 -> 45.5 us).
 template <int DIM, int N, int M, typename R, bool RK, int NV>
 __host__ __device__ constexpr bool rhs_par_dirs() {
     return TRIXI_HIP_PAR_DIRS != 0 && DIM > 1 && (M * cpow(N, DIM - 1)) % 64 == 0 &&
