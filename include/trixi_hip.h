@@ -354,10 +354,11 @@ int trixi_hip_advance_f32(trixi_hip_ctx* ctx, float* u, float* k, double* t, dou
  * the scalar is on the host.  No counterpart in the reference: it is for
  * callers that cannot allocate device memory (tight time-stepping loops,
  * harnesses that forbid hipMalloc).
- * Limit: at most 2047 block partials (the grid is at most 1024 blocks of 256
- * elements, so every mesh fits); larger grids are rejected with
- * TRIXI_HIP_EINVAL.  All calls on one GPU share the scratch: calls that
- * overlap on one GPU (several host threads or streams) race. */
+ * Limit: at most 2047 block partials (the grid is at most 1024 blocks, each
+ * taking 16 elements at a time, so every mesh fits); larger grids are rejected
+ * with TRIXI_HIP_EINVAL.  All calls on one GPU share the scratch: the results of
+ * calls that overlap on one GPU (several host threads or streams) are
+ * undefined; later calls are not affected. */
 int trixi_hip_max_dt_noalloc(trixi_hip_ctx* ctx, const double* u, double* max_dt,
                              trixi_hip_stream stream);
 

@@ -11,6 +11,7 @@
 // 2950 us, integrals 104, max_dt 23; at 32768 elements max_dt 47 + 13.
 #pragma once
 
+#include "arrival.hpp"
 #include "initial_conditions.hpp"
 #include "physics.hpp"
 
@@ -26,9 +27,9 @@ __device__ __forceinline__ void store_partial(double* p, double x) {
 }
 
 // Combines the blocks' partial vectors (m components, the first nsum summed,
-// the others their maximum) in the last block to arrive, which writes `out` and
-// leaves `arrived` at zero for the next call.  Every thread of every block calls
-// it after its block's store_partial calls.
+// the others their maximum) in the last block to arrive, which writes `out`; the
+// count in `arrived` wraps to zero there (arrival.hpp).  Every thread of every
+// block calls it after its block's store_partial calls.
 // Returns true in the last block's thread 0, with component 0 in `first`.
 template <int THREADS>
 __device__ __forceinline__ bool finish_partials(const double* partial, double* out, unsigned* arrived, int m,
@@ -37,7 +38,7 @@ __device__ __forceinline__ bool finish_partials(const double* partial, double* o
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's partials have arrived
     __syncthreads();
     if (threadIdx.x == 0)
-        last = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+        last = arrival_is_last(atomicInc(arrived, gridDim.x - 1), gridDim.x);
     __syncthreads();
     if (!last) return false;
     asm volatile("" ::: "memory");
@@ -67,7 +68,6 @@ __device__ __forceinline__ bool finish_partials(const double* partial, double* o
         if (lane == 0) out[c] = x;
         if (c == 0) first = x;
     }
-    if (threadIdx.x == 0) __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return threadIdx.x == 0;
 }
 template <int THREADS>

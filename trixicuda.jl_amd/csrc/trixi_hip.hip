@@ -731,7 +731,7 @@ struct trixi_hip_ctx {
     double* d_time = nullptr;
     double* d_partial = nullptr;
     double* h_result = nullptr;    // pinned: the last block of a reduction writes here
-    unsigned* d_arrived = nullptr;  // blocks of a running reduction that have arrived
+    unsigned* d_arrived = nullptr;  // blocks of a running reduction that have arrived [ARRIVAL_COUNTERS]
     double* d_Vinv = nullptr;
     double* d_Vdm = nullptr;
     double* d_wa = nullptr;
@@ -1166,12 +1166,12 @@ int trixi_hip_create(const trixi_hip_config* config, const trixi_hip_mesh* mesh,
     ALLOC(c->d_alpha, E * sizeof(double));
     ALLOC(c->d_time, TIME_DOUBLES * sizeof(double));
     ALLOC(c->d_partial, (size_t)c->nblocks_red * 18 * sizeof(double));
-    ALLOC(c->d_arrived, sizeof(unsigned));
+    ALLOC(c->d_arrived, ARRIVAL_COUNTERS * sizeof(unsigned));
     ALLOC(c->d_consts, sizeof(RhsConst));
     c->h_result = take_result_slot();
     if (!c->h_result)
         return cleanup_fail(TRIXI_HIP_ENOMEM, "hipHostMalloc failed for the reduction results");
-    if (hipMemset(c->d_arrived, 0, sizeof(unsigned)) != hipSuccess)
+    if (hipMemset(c->d_arrived, 0, ARRIVAL_COUNTERS * sizeof(unsigned)) != hipSuccess)
         return cleanup_fail(TRIXI_HIP_EDEVICE, "hipMemset failed in create");
     ALLOC(c->d_Vinv, N * N * sizeof(double));
     ALLOC(c->d_Vdm, c->NA * N * sizeof(double));
@@ -1576,11 +1576,13 @@ static int reduction_blocks(const trixi_hip_ctx* c) {
 }
 
 // The largest scaled wave speed of u (of type S) into `result`, which the
-// device writes, with the block partials in `partial` (at least `blocks`
-// doubles) and the arrival count in `arrived` (zero before and after).
+// device writes, with the block partials in `partial` (reduction_blocks
+// doubles).
 extern "C++" template <typename S>
-static int launch_max_speed(trixi_hip_ctx* ctx, const S* u, hipStream_t s, int blocks, double* partial,
-                            double* result, unsigned* arrived, const StepControl& step = StepControl{}) {
+static int launch_max_speed(trixi_hip_ctx* ctx, const S* u, hipStream_t s, double* partial, double* result,
+                            const StepControl& step = StepControl{}) {
+    const int blocks = reduction_blocks(ctx);
+    unsigned* const arrived = ctx->d_arrived + ARRIVED_ELEMENTS;
     const PhysParams& P = ctx->consts.phys;
     const int eq = ctx->cfg.equation, dim = ctx->dim;
 #define MS(EQT, D)                                                                                                 \
@@ -1619,7 +1621,7 @@ static int launch_max_speed(trixi_hip_ctx* ctx, const S* u, hipStream_t s, int b
 
 extern "C++" template <typename S>
 static int max_dt_any(trixi_hip_ctx* ctx, const S* u, double* max_dt, hipStream_t s) {
-    int rc = launch_max_speed(ctx, u, s, reduction_blocks(ctx), ctx->d_partial, ctx->h_result, ctx->d_arrived);
+    int rc = launch_max_speed(ctx, u, s, ctx->d_partial, ctx->h_result);
     if (rc) return rc;
     HIP_TRY(hipStreamSynchronize(s));
     *max_dt = max_dt_of(ctx->N, ctx->h_result[0]);
@@ -1641,20 +1643,20 @@ int trixi_hip_max_dt_noalloc(trixi_hip_ctx* ctx, const double* u, double* max_dt
     if (!ctx || !u || !max_dt) return fail(TRIXI_HIP_EINVAL, "null argument");
     // the same grid as trixi_hip_max_dt: the same partials and maximum
     const int blocks = reduction_blocks(ctx);
-    if (blocks + 2 > TRIXI_HIP_SCRATCH_DOUBLES)
+    if (blocks + 1 > TRIXI_HIP_SCRATCH_DOUBLES)
         return fail(TRIXI_HIP_EINVAL, "max_dt_noalloc: " + std::to_string(blocks) +
                                           " block partials exceed the static scratch of " +
-                                          std::to_string(TRIXI_HIP_SCRATCH_DOUBLES - 2));
+                                          std::to_string(TRIXI_HIP_SCRATCH_DOUBLES - 1));
     double* sp = nullptr;
     int rc = scratch_ptr(&sp);
     if (rc) return rc;
-    // partials in [0, blocks), the arrival count and the maximum in the last
-    // two slots; every partial is written before it is read, and the count is
-    // zero at load and left at zero, so nothing needs clearing between calls
+    // partials in [0, blocks), the maximum in the last slot; every partial is
+    // written before it is read, so nothing needs clearing between calls.  The
+    // arrival count is the context's own: in the scratch, contexts of other grid
+    // sizes would share it, and calls that overlap would leave it wrong.
     hipStream_t s = (hipStream_t)stream;
     double* const result = sp + TRIXI_HIP_SCRATCH_DOUBLES - 1;
-    rc = launch_max_speed(ctx, u, s, blocks, sp, result,
-                          reinterpret_cast<unsigned*>(sp + TRIXI_HIP_SCRATCH_DOUBLES - 2));
+    rc = launch_max_speed(ctx, u, s, sp, result);
     if (rc) return rc;
     double m = 0.0;
     HIP_TRY(hipMemcpyAsync(&m, result, sizeof(double), hipMemcpyDeviceToHost, s));
@@ -1690,8 +1692,7 @@ static int advance_any(trixi_hip_ctx* c, S* u, S* k, double* t, double t_end, do
         for (int64_t i = 0; i < chunk; ++i) {
             q.log = c->h_result + kLog + 2 * i;
             if (cfl > 0.0) {
-                int rc = launch_max_speed(c, (const S*)u, s, reduction_blocks(c), c->d_partial, c->h_result,
-                                          c->d_arrived, q);
+                int rc = launch_max_speed(c, (const S*)u, s, c->d_partial, c->h_result, q);
                 if (rc) return rc;
             } else {
                 hipLaunchKernelGGL(next_step_kernel, dim3(1), dim3(1), 0, s, q, dt);
@@ -1748,8 +1749,8 @@ static hipError_t launch_error_norms(trixi_hip_ctx* ctx, const double* u, const 
     const bool wave = q.ic == TRIXI_HIP_IC_CONVERGENCE_TEST;
 #define TRIXI_HIP_EN(X)                                                                                             \
     hipLaunchKernelGGL((error_norms_kernel<DIM, N, X>), dim3(blocks), dim3(64 * waves), (unsigned)(waves * wave_bytes), \
-                       s, u, ctx->d_x, ctx->d_invJ, ctx->d_partial, ctx->h_result, ctx->d_arrived, ctx->d_Vdm,        \
-                       ctx->d_wa, ctx->E, q, t, ctx->nv)
+                       s, u, ctx->d_x, ctx->d_invJ, ctx->d_partial, ctx->h_result, ctx->d_arrived + ARRIVED_NORMS,    \
+                       ctx->d_Vdm, ctx->d_wa, ctx->E, q, t, ctx->nv)
     if (wave && q.eq == EQ_EULER)
         TRIXI_HIP_EN(EN_EULER_WAVE);
     else if (wave && q.eq == EQ_LINADV)
@@ -1797,7 +1798,7 @@ int trixi_hip_integrate(trixi_hip_ctx* ctx, const double* u, double* integral, t
     hipStream_t s = (hipStream_t)stream;
 #define IK(D, NQ)                                                                                                  \
     hipLaunchKernelGGL((integrate_kernel<D, NQ>), dim3(reduction_blocks(ctx)), dim3(RED_THREADS), 0, s, u, ctx->d_invJ, \
-                       ctx->d_partial, ctx->h_result, ctx->d_arrived, ctx->d_w, ctx->E, ctx->nv)
+                       ctx->d_partial, ctx->h_result, ctx->d_arrived + ARRIVED_ELEMENTS, ctx->d_w, ctx->E, ctx->nv)
 #define IKN(NQ)                                                                    \
     case NQ:                                                                       \
         if (ctx->dim == 1) IK(1, NQ); else if (ctx->dim == 2) IK(2, NQ); else IK(3, NQ); \
@@ -2070,7 +2071,8 @@ int trixi_hip_check_state(trixi_hip_ctx* ctx, const double* u, int32_t* flags, i
     const int threads = 256;
     const int blocks = (int)std::min<int64_t>((ctx->E + threads - 1) / threads, ctx->nblocks_red);
     hipLaunchKernelGGL(check_state_kernel, dim3(blocks), dim3(threads), 0, s, u, flags, ctx->d_partial,
-                       ctx->h_result, ctx->d_arrived, ctx->cfg.equation, ctx->dim, ctx->nv, ctx->nn, ctx->E, ctx->consts.phys);
+                       ctx->h_result, ctx->d_arrived + ARRIVED_STATE, ctx->cfg.equation, ctx->dim, ctx->nv, ctx->nn,
+                       ctx->E, ctx->consts.phys);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s));
     *nbad = (int64_t)ctx->h_result[0];
