@@ -338,7 +338,9 @@ int trixi_hip_max_dt_f32(trixi_hip_ctx* ctx, const float* u, double* max_dt,
  * cfl > 0, else of size dt, the last one shortened to end at t_end.  *t and
  * *nsteps return the time reached and the steps taken; blocks until they are on
  * the host, but not between the steps (max_dt, the stage times and the end of
- * the run stay on the device).  Replaces the reference's solve loop with a
+ * the run stay on the device).  An error ends the run: the steps queued before it
+ * have ended then, u is the state at *t after *nsteps steps and k undefined (after
+ * an error of the device itself both are).  Replaces the reference's solve loop with a
  * StepsizeCallback (examples/euler_ec_3d.jl:45-55). */
 int trixi_hip_advance(trixi_hip_ctx* ctx, double* u, double* k, double* t, double t_end,
                       double cfl, double dt, int64_t max_steps, int64_t* nsteps,

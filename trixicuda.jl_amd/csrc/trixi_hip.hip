@@ -17,6 +17,7 @@
 #include "initial_conditions.hpp"
 #include "indicator.hpp"
 #include "reductions.hpp"
+#include "time_loop.hpp"
 
 namespace trixi_hip {
 
@@ -1669,8 +1670,9 @@ int trixi_hip_max_dt_noalloc(trixi_hip_ctx* ctx, const double* u, double* max_dt
 // synchronisation per step: the wave-speed reduction (or, with a fixed dt, a
 // kernel of one thread) leaves the step's times on the device for the stages and
 // logs the step in pinned memory; the host queues a chunk of steps, waits once
-// and reads the log.  A step past the end does nothing (RhsArgs::done), so a
-// chunk may be longer than what is left.
+// and reads the log (time_loop.hpp).  A step past the end does nothing
+// (RhsArgs::done), so a chunk may be longer than what is left; u is written by a
+// step's last launch only, so that a step that could not be queued whole leaves it.
 extern "C++" template <typename S>
 static int advance_any(trixi_hip_ctx* c, S* u, S* k, double* t, double t_end, double cfl, double dt,
                        int64_t max_steps, int64_t* nsteps, hipStream_t s) {
@@ -1680,38 +1682,25 @@ static int advance_any(trixi_hip_ctx* c, S* u, S* k, double* t, double t_end, do
     q.cfl = cfl;
     q.N = c->N;
     for (int st = 0; st < 5; ++st) q.c[st] = CK_C[st];
+    *nsteps = 0;
     hipLaunchKernelGGL(start_time_kernel, dim3(1), dim3(1), 0, s, c->d_time, *t);
     HIP_TRY(hipGetLastError());
-    double h = cfl > 0.0 ? 0.0 : dt;  // last step size: how many steps are left at most a guess
-    int64_t done = 0;
-    while (*t < t_end && done < max_steps) {
-        // by the last step size, two where there is none yet
-        const double left = h > 0.0 ? ceil((t_end - *t) / h) : 2.0;
-        int64_t chunk = std::min<int64_t>(kChunk, max_steps - done);
-        if (left < (double)chunk) chunk = left > 1.0 ? (int64_t)left : 1;
-        for (int64_t i = 0; i < chunk; ++i) {
-            q.log = c->h_result + kLog + 2 * i;
-            if (cfl > 0.0) {
-                int rc = launch_max_speed(c, (const S*)u, s, c->d_partial, c->h_result, q);
-                if (rc) return rc;
-            } else {
-                hipLaunchKernelGGL(next_step_kernel, dim3(1), dim3(1), 0, s, q, dt);
-                HIP_TRY(hipGetLastError());
-            }
-            int rc = enqueue_rk_stages(c, u, k, s, c->d_time + TIME_DONE);
+    auto queue = [&](int64_t i) -> int {
+        q.log = c->h_result + kLog + 2 * i;
+        if (cfl > 0.0) {
+            int rc = launch_max_speed(c, (const S*)u, s, c->d_partial, c->h_result, q);
             if (rc) return rc;
+        } else {
+            hipLaunchKernelGGL(next_step_kernel, dim3(1), dim3(1), 0, s, q, dt);
+            HIP_TRY(hipGetLastError());
         }
+        return enqueue_rk_stages(c, u, k, s, c->d_time + TIME_DONE);
+    };
+    auto wait = [&]() -> int {
         HIP_TRY(hipStreamSynchronize(s));
-        for (int64_t i = 0; i < chunk; ++i) {
-            const double* log = c->h_result + kLog + 2 * i;
-            if (log[1] < 0.0) break;
-            *t = log[0];
-            h = log[1];
-            ++done;
-            *nsteps = done;
-        }
-    }
-    return TRIXI_HIP_OK;
+        return TRIXI_HIP_OK;
+    };
+    return run_steps(t, t_end, cfl > 0.0 ? 0.0 : dt, max_steps, kChunk, c->h_result + kLog, nsteps, queue, wait);
 }
 
 static int check_advance(const trixi_hip_ctx* c, const void* u, const void* k, const double* t, double cfl, double dt,
@@ -1727,7 +1716,6 @@ int trixi_hip_advance(trixi_hip_ctx* ctx, double* u, double* k, double* t, doubl
     int rc = check_advance(ctx, u, k, t, cfl, dt, nsteps);
     if (rc) return rc;
     if (fp32_state(ctx)) return fail(TRIXI_HIP_EINVAL, "this context's state is FP32: use trixi_hip_advance_f32");
-    *nsteps = 0;
     return advance_any(ctx, u, k, t, t_end, cfl, dt, max_steps, nsteps, (hipStream_t)stream);
 }
 
@@ -1736,7 +1724,6 @@ int trixi_hip_advance_f32(trixi_hip_ctx* ctx, float* u, float* k, double* t, dou
     int rc = check_advance(ctx, u, k, t, cfl, dt, nsteps);
     if (rc) return rc;
     if (!fp32_state(ctx)) return fail(TRIXI_HIP_EINVAL, "this context's state is FP64: use trixi_hip_advance");
-    *nsteps = 0;
     return advance_any(ctx, u, k, t, t_end, cfl, dt, max_steps, nsteps, (hipStream_t)stream);
 }
 
