@@ -82,9 +82,16 @@ def advance(u, k, t, t_end, semi, cfl=0.0, dt=0.0, max_steps=10**7, stream=None)
     s = stream if stream is not None else torch.cuda.current_stream()
     tt, n = ctypes.c_double(t), ctypes.c_int64()
     fn = L.lib().trixi_hip_advance_f32 if semi.fp32_state else L.lib().trixi_hip_advance
-    L.check(fn(semi.ctx, _ptr(u), _ptr(k), ctypes.byref(tt), float(t_end), float(cfl), float(dt), int(max_steps),
-               ctypes.byref(n), ctypes.c_void_p(s.cuda_stream)))
+    L.check(fn(semi.ctx, _ptr(u), _ptr(k), ctypes.byref(tt), float(t_end), float(cfl), float(dt),
+               int(min(max_steps, 2**63 - 1)), ctypes.byref(n), ctypes.c_void_p(s.cuda_stream)))
     return tt.value, n.value
+
+
+def _steps_to_queue(nsteps, maxiters, intervals):
+    """Steps of one native run from step nsteps on: while nsteps < maxiters (which
+    may be fractional or infinite), up to the next multiple of an interval."""
+    left = [maxiters - nsteps, 2**31] + [i - nsteps % i for i in intervals if i > 0]
+    return max(1, int(min(left)))
 
 
 def solve(ode, alg=None, dt=None, callback=(), use_graph=True, maxiters=10**7):
@@ -107,14 +114,14 @@ def solve(ode, alg=None, dt=None, callback=(), use_graph=True, maxiters=10**7):
     t, nsteps, h = t0, 0, 0.0
     # steps without host work between them run as one native loop: nothing to
     # save, and analysis only at known step numbers
-    cfl = stepsize.cfl if type(stepsize) is StepsizeCallback else 0.0
+    plain = type(stepsize) is StepsizeCallback and "dt" not in vars(stepsize)
     native = not saves and all(type(a) is AnalysisCallback for a in analysis) and (
-        cfl > 0.0 if stepsize is not None else dt > 0.0)
+        plain and stepsize.cfl > 0.0 if stepsize is not None else dt > 0.0)
     with torch.cuda.stream(stream):
         while native and t < t1 and nsteps < maxiters:
-            todo = min([maxiters - nsteps] + [a.interval - nsteps % a.interval for a in analysis if a.interval > 0])
-            t, n = advance(u, k, t, t1, semi, cfl=cfl, dt=0.0 if stepsize is not None else dt, max_steps=todo,
-                           stream=stream)
+            t, n = advance(u, k, t, t1, semi, cfl=stepsize.cfl if stepsize is not None else 0.0,
+                           dt=0.0 if stepsize is not None else dt, stream=stream,
+                           max_steps=_steps_to_queue(nsteps, maxiters, [a.interval for a in analysis]))
             nsteps += n
             for a in analysis:
                 a(u, t, nsteps)
