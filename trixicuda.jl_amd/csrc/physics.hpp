@@ -1222,14 +1222,42 @@ struct GlmMhd {
         f[8] = P.c_h * B[o];
     }
 
+    // The argument of the fast speed's inner root, (a2 + b2)^2 - 4 a2 bo2 with
+    // b2 = bo2 + bt2 (the field along and across the direction).  It is zero where
+    // the field lies along the direction and a2 = b2, and the difference then rounds
+    // below zero (in half of such states with a fused multiply-add), whose root is
+    // NaN.  FP64: as a sum of squares.  FP32 arithmetic: the difference, kept from
+    // falling below zero (the sum takes more registers than the spilling kernels on
+    // refined meshes have: 3D RK stage at 4544 elements 106.5 -> 112 us).
+    template <typename R>
+    __device__ static R fast_root2(R a2, R b2, R bo2, R bt2) {
+        if constexpr (std::is_same<R, double>::value) {
+            const R d = a2 - b2;
+            return d * d + R(4) * a2 * bt2;
+        } else {
+            const R s = a2 + b2;
+            return dmax(s * s - R(4) * a2 * bo2, R(0));  // (a NaN stays)
+        }
+    }
+    // |B|^2 across direction o
+    template <typename R>
+    __device__ static R transverse2(const R* B, int o) {
+        R t = R(0);
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+            if (d != o) t += B[d] * B[d];
+        return t;
+    }
     template <typename R, typename L>
     __device__ static R fast_speed(const Node<R, L>& n, int o, const PhysR<R>& P) {
         const R inv_rho = rdiv(R(1), n.rho);
         const R a_square = P.gamma * n.p * inv_rho;
-        const R b_square = (n.B[0] * n.B[0] + n.B[1] * n.B[1] + n.B[2] * n.B[2]) * inv_rho;
-        const R bo2 = n.B[o] * n.B[o] * inv_rho;
-        const R s = a_square + b_square;
-        return rsqrt_(R(0.5) * s + R(0.5) * rsqrt_(s * s - R(4) * a_square * bo2));
+        const R t = transverse2(n.B, o);
+        const R b_square = (std::is_same<R, double>::value
+                                ? n.B[o] * n.B[o] + t
+                                : n.B[0] * n.B[0] + n.B[1] * n.B[1] + n.B[2] * n.B[2]) * inv_rho;
+        const R D = fast_root2(a_square, b_square, n.B[o] * n.B[o] * inv_rho, t * inv_rho);
+        return rsqrt_(R(0.5) * (a_square + b_square) + R(0.5) * rsqrt_(D));
     }
 
     // Roe-averaged normal velocity and fast magnetoacoustic speed (Cargo &
@@ -1243,7 +1271,7 @@ struct GlmMhd {
         const R sl = rsqrt_(l.rho), sr = rsqrt_(r.rho);
         const R inv_add = rdiv(R(1), sl + sr), inv_prod = rdiv(R(1), sl * sr);
         const R wl = sl * inv_add, wr = sr * inv_add;
-        R v2 = R(0), B2 = R(0), dB2 = R(0), Bo = R(0);
+        R v2 = R(0), B2 = R(0), Bt2 = R(0), dB2 = R(0), Bo = R(0);
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
             const R vd = l.v[d] * wl + r.v[d] * wr;
@@ -1255,6 +1283,8 @@ struct GlmMhd {
             if (d == o) {
                 vel = vd;
                 Bo = Bd;
+            } else {
+                Bt2 += Bd * Bd;
             }
         }
         const R mbl = l.B[0] * l.B[0] + l.B[1] * l.B[1] + l.B[2] * l.B[2];
@@ -1262,10 +1292,9 @@ struct GlmMhd {
         const R Hl = rdiv(l.cons(4) + l.p + R(0.5) * mbl, l.rho), Hr = rdiv(r.cons(4) + r.p + R(0.5) * mbr, r.rho);
         const R H = Hl * wl + Hr * wr;
         const R X = R(0.5) * dB2 * inv_add * inv_add;
-        const R b2 = B2 * inv_prod;
+        const R b2 = (std::is_same<R, double>::value ? Bo * Bo + Bt2 : B2) * inv_prod;
         const R a2 = (R(2) - P.gamma) * X + P.gm1 * (H - R(0.5) * v2 - b2);
-        const R ca = Bo * Bo * inv_prod;
-        const R astar = rsqrt_((a2 + b2) * (a2 + b2) - R(4) * a2 * ca);
+        const R astar = rsqrt_(fast_root2(a2, b2, Bo * Bo * inv_prod, Bt2 * inv_prod));
         cf = rsqrt_(R(0.5) * (a2 + b2 + astar));
     }
 
@@ -1319,8 +1348,7 @@ struct GlmMhd {
     // Local Lax-Friedrichs in FP64.  The physical flux is v_o u plus pressure
     // and magnetic terms (B_o and psi: c_h psi and c_h B_o alone), so that
     //   2 f = v_l,o u_l + v_r,o u_r + lambda (u_l - u_r) + those terms,
-    // with |B|^2 shared by the fluxes, the states and the fast speeds, for which
-    //   c_f^2 = (S + sqrt(S^2 - 4 gamma p B_o^2)) / (2 rho),  S = gamma p + |B|^2.
+    // with |B|^2 shared by the fluxes, the states and the fast speeds.
     // (The interfaces are the heaviest part of the MHD kernel: 3D rhs! at 4096
     // elements 23.8 -> 23.3 us against two fluxes and two states.)
     template <int KIND, typename L>
@@ -1332,8 +1360,8 @@ struct GlmMhd {
         for (int k = 0; k < 2; ++k) {
             const double* v = n[k]->v;
             const double* B = n[k]->B;
-            const double psi = n[k]->psi, p = n[k]->p, gp = P.gamma * p;
-            const double b2 = fma(B[2], B[2], fma(B[1], B[1], B[0] * B[0]));
+            const double psi = n[k]->psi, p = n[k]->p;
+            const double bt2 = transverse2(B, o), b2 = fma(B[o], B[o], bt2);
             u[k][0] = n[k]->rho;
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
@@ -1348,9 +1376,8 @@ struct GlmMhd {
             cB[k] = P.c_h * B[o];
             const double vB = fma(v[2], B[2], fma(v[1], B[1], v[0] * B[0]));
             en[k] = fma(v[o], e + pt[k], fma(psi, cB[k], -(B[o] * vB)));
-            const double S = gp + b2;
-            const double D = fma(S, S, -4.0 * gp * (B[o] * B[o]));
-            c[k] = rsqrt_(0.5 * (S + rsqrt_(D)) * rdiv(1.0, n[k]->rho));
+            const double ir = rdiv(1.0, n[k]->rho), as = P.gamma * p * ir, bs = b2 * ir;
+            c[k] = rsqrt_(0.5 * (as + bs + rsqrt_(fast_root2(as, bs, 0.0, bt2 * ir))));
         }
         double lam;
         if (KIND == FLUX_LLF_NAIVE)
@@ -1480,7 +1507,7 @@ struct GlmMhd {
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
             const R s = a_square + b_square;
-            const R cf = sqrt(R(0.5) * s + R(0.5) * sqrt(s * s - R(4) * a_square * bb[d] * bb[d]));
+            const R cf = sqrt(R(0.5) * s + R(0.5) * sqrt(fast_root2(a_square, b_square, R(0), transverse2(bb, d))));
             lam[d] = dabs(vv[d]) + cf;
         }
     }
