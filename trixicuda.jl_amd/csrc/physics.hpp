@@ -114,7 +114,10 @@ __device__ __forceinline__ int64_t soa(int v, int node, int64_t e, int64_t slab,
 //         residual step (within about 1 ulp, far inside the FP64 parity
 //         bound, 6 instructions instead of the 11-instruction IEEE sequence);
 //         square root = v_rsq_f64 with one coupled (Goldschmidt) step and one
-//         residual correction (within 1 ulp; 0 and infinity as they are).
+//         residual correction (measured over 2^18 arguments per range: correctly
+//         rounded from 2^-1000 up, within 1 ulp down to the smallest normal
+//         number, relative error 4e-15 of subnormal ones, whose residual is lost;
+//         0 and infinity as they are).
 //   FP32 (mixed mode): v_rcp_f32 and v_sqrt_f32 (within 2 ulp of FP32).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ double rrcp(double d) {
@@ -191,14 +194,14 @@ __device__ __forceinline__ R inv_ln_mean_logs(R x, R y, L lx, L ly) {
 
 // ---------------------------------------------------------------------------
 // The two logarithmic means of an entropy-conservative flux without node
-// logarithms (FP64 arithmetic): ln_mean(x1, y1) and inv_ln_mean(x2, y2) with
-// one reciprocal for both, from the series in z^2, z = (y - x) / (x + y).
+// logarithms (FP64 arithmetic): ln_mean(x1, y1) and inv_ln_mean(x2, y2) from
+// the series in z^2, z = (y - x) / (x + y).
 //   log(y / x) = z P(z^2), P(q) = 2 atanh(sqrt q) / sqrt q, and Q = 1 / P:
 //   minimax polynomials of degree 6 for |z| < 0.15 (y / x < 1.353), relative
-//   error below 3e-17 (P) and 6e-18 (Q), so the result is the mean's to
-//   round-off.
-// MEANS_NEAR: the caller knows that |z| < 0.15 for both.  MEANS_ANY: any
-// x, y; lanes further apart take the closed form with the logarithm of the
+//   error of the stored coefficients below 5.2e-17 (P) and 1.1e-17 (Q), less than
+//   half a unit in the last place.
+// MEANS_NEAR: the caller knows that |z| < 0.15 for both (near_line).  MEANS_ANY:
+// any x, y; lanes further apart take the closed form with the logarithm of the
 // quotient, in a block that a wave without such lanes skips.
 // Against node logarithms (two per node, staged in LDS) with a three-term
 // series below |z| = 0.01, the FP64 kernels drop the logarithms, their LDS and
@@ -221,13 +224,34 @@ __device__ __forceinline__ double raw_max(double x, double y) {
 // y / x < 1.15 / 0.85 for x <= y (false for x <= 0 and for NaN)
 __device__ __forceinline__ bool near_ratio(double x, double y) { return 0.85 * y < 1.15 * x; }
 
+// 1 / s1 and 1 / s2 of the sums of two means, MEANS_NEAR from one reciprocal of
+// their product (rho^2 p in size, which near_range keeps inside the FP64 range; two
+// reciprocals take 0.5 us more of 80 in 3D at 32768 elements and 0.3 of 22 in 2D).
+template <int MEANS>
+__device__ __forceinline__ void sum_reciprocals(double s1, double s2, double& r1, double& r2) {
+    if constexpr (MEANS == MEANS_NEAR) {
+        const double r = rrcp(s1 * s2);
+        r1 = r * s2;
+        r2 = r * s1;
+    } else {
+        r1 = rrcp(s1);
+        r2 = rrcp(s2);
+    }
+}
+// whether the products s1 s2 of a line whose ratios are near lie well inside the
+// FP64 range, by one of its nodes (the others' within a factor of 20)
+__device__ __forceinline__ bool near_range(double rho, double p) {
+    const double w = rho * (rho * p);
+    return w > 0x1p-960 && w < 0x1p960;
+}
+
 template <int MEANS>
 __device__ __forceinline__ void log_free_means(double x1, double y1, double x2, double y2, double& mean1,
                                                double& inv_mean2) {
     const double s1 = x1 + y1, d1 = y1 - x1;
     const double s2 = x2 + y2, d2 = y2 - x2;
-    const double r = rrcp(s1 * s2);
-    const double r1 = r * s2, r2 = r * s1;
+    double r1, r2;
+    sum_reciprocals<MEANS>(s1, s2, r1, r2);
     const double z1 = d1 * r1, z2 = d2 * r2;
     const double q1 = z1 * z1, q2 = z2 * z2;
     double Q = fma(q1, fastlog_const<true>(-0.008948152998574805), fastlog_const<true>(-0.01088099532782093));
@@ -596,7 +620,7 @@ struct Euler {
             p0 = raw_min(p0, n[i].p);
         }
         const bool a = near_ratio(r0, r1), b = near_ratio(c0 * c0, c1 * c1), c = p0 > 0.0;
-        return a && b && c;
+        return a && b && c && near_range(n[0].rho, n[0].p);
     }
 
     template <int KIND, typename R, typename L>
@@ -1420,7 +1444,7 @@ struct GlmMhd {
             b1 = raw_max(b1, b);
         }
         const bool a = near_ratio(r0, r1), b = near_ratio(b0, b1);
-        return a && b;
+        return a && b && near_range(n[0].rho, n[0].p);
     }
 
     template <int KIND, typename R, typename L>

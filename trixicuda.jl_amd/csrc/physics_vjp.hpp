@@ -80,8 +80,8 @@ __device__ __forceinline__ void log_free_mean_grads(double x1, double y1, double
                                                     double& Ly, double& I, double& Ix, double& Iy) {
     const double s1 = x1 + y1, d1 = y1 - x1;
     const double s2 = x2 + y2, d2 = y2 - x2;
-    const double r = rrcp(s1 * s2);
-    const double r1 = r * s2, r2 = r * s1;
+    double r1, r2;
+    sum_reciprocals<MEANS>(s1, s2, r1, r2);
     const double z1 = d1 * r1, z2 = d2 * r2;
     const double q1 = z1 * z1, q2 = z2 * z2;
     double Q = fastlog_const<true>(-0.007279622637948864), Qd = Q;
