@@ -219,7 +219,7 @@ __global__ void __launch_bounds__((group_threads<DIM, N, M>()), WAVES) rhs_group
                 for (int f = 0; f < 2 * DIM; ++f) {
                     if (EXT && nb[f] < 0) {
                         if (nb[f] == -1) continue;  // boundary: no neighbour
-                        const int32_t* mn = kc.mnb + (int64_t)(-2 - nb[f]) * kc.mK;
+                        const int32_t* mn = in_global(kc.mnb) + (int64_t)(-2 - nb[f]) * kc.mK;
                         for (int k = 0; k < kc.mK; ++k)
                             if (mn[k] >= 0) alpha = dmax(alpha, 0.5 * a.alpha_raw[mn[k]]);
                         continue;
@@ -408,12 +408,12 @@ __global__ void __launch_bounds__((group_threads<DIM, N, M>()), WAVES) rhs_group
                 }
                 constexpr double h = TW ? 2.0 : 1.0;
                 if (nm <= -2) {
-                    const double* mf = kc.mflux + ((int64_t)(-2 - nm) * NL + line) * NV;
+                    const double* mf = in_global(kc.mflux) + ((int64_t)(-2 - nm) * NL + line) * NV;
 #pragma unroll
                     for (int v = 0; v < NV; ++v) fm[v] = h * mf[Rot::variable(v, o)];
                 }
                 if (np <= -2) {
-                    const double* mf = kc.mflux + ((int64_t)(-2 - np) * NL + line) * NV;
+                    const double* mf = in_global(kc.mflux) + ((int64_t)(-2 - np) * NL + line) * NV;
 #pragma unroll
                     for (int v = 0; v < NV; ++v) fp[v] = h * mf[Rot::variable(v, o)];
                 }

@@ -132,6 +132,17 @@ using RhsConstArg = std::conditional_t<std::is_same<R, double>::value, const Rhs
 __device__ __forceinline__ const RhsConst& consts_of(const RhsConst* p) { return *p; }
 __device__ __forceinline__ const RhsConst& consts_of(const RhsConst& v) { return v; }
 
+// A pointer read from the constants, known to point to global memory (as one that is
+// a kernel argument is): its loads are otherwise flat ones, which wait for LDS too.
+template <typename T>
+__device__ __forceinline__ const T* in_global(const T* p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return (const T*)(const __attribute__((address_space(1))) T*)(uintptr_t)p;
+#else
+    return p;
+#endif
+}
+
 struct RhsArgs {
     // state vectors of the kernel's state type S (double, or float for the
     // FP32-state precision)
@@ -164,7 +175,7 @@ template <int DIM, int NN, int NV, typename R>
 __device__ __forceinline__ void boundary_state(const RhsArgs& a, const RhsConst& kc, int64_t e, int node, double t, R* ub) {
     double xx[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-    for (int d = 0; d < DIM; ++d) xx[d] = kc.x[((int64_t)d * NN + node) * a.E + e];
+    for (int d = 0; d < DIM; ++d) xx[d] = in_global(kc.x)[((int64_t)d * NN + node) * a.E + e];
     double uu[5];
     boundary_value(kc.bc_ic, xx, t, uu);
 #pragma unroll
@@ -178,7 +189,7 @@ template <int DIM, int NN, int NV>
 __device__ __forceinline__ void source_at(const RhsArgs& a, const RhsConst& kc, int64_t e, int node, double t, double* sv) {
     double xx[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-    for (int d = 0; d < DIM; ++d) xx[d] = kc.x[((int64_t)d * NN + node) * a.E + e];
+    for (int d = 0; d < DIM; ++d) xx[d] = in_global(kc.x)[((int64_t)d * NN + node) * a.E + e];
     if constexpr (NV == 1) {
         sv[0] = source_burgers_convergence_test(xx[0], t);
         return;
@@ -468,7 +479,7 @@ rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
                     // boundary faces have no neighbour; a mortar face has the
                     // elements on the other side of the mortar
                     if (nb[s] == -1) continue;
-                    const int32_t* mn = kc.mnb + (int64_t)(-2 - nb[s]) * kc.mK;
+                    const int32_t* mn = in_global(kc.mnb) + (int64_t)(-2 - nb[s]) * kc.mK;
                     for (int k = 0; k < kc.mK; ++k) {
                         if (mn[k] < 0) continue;
                         const double an = 0.5 * a.alpha_raw[mn[k]];
@@ -763,12 +774,12 @@ rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
             if constexpr (EXT) {
                 // mortar faces: the face node of this line is `line`
                 if (nb[2 * d] <= -2) {
-                    const double* mf = kc.mflux + ((int64_t)(-2 - nb[2 * d]) * NL + line) * NV;
+                    const double* mf = in_global(kc.mflux) + ((int64_t)(-2 - nb[2 * d]) * NL + line) * NV;
 #pragma unroll
                     for (int v = 0; v < NV; ++v) fm[v] = (TW ? R(2) : R(1)) * (R)mf[v];
                 }
                 if (nb[2 * d + 1] <= -2) {
-                    const double* mf = kc.mflux + ((int64_t)(-2 - nb[2 * d + 1]) * NL + line) * NV;
+                    const double* mf = in_global(kc.mflux) + ((int64_t)(-2 - nb[2 * d + 1]) * NL + line) * NV;
 #pragma unroll
                     for (int v = 0; v < NV; ++v) fp[v] = (TW ? R(2) : R(1)) * (R)mf[v];
                 }
@@ -1216,7 +1227,7 @@ rhs_np_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
         double* const buf = ind_buf;
         double* const e2 = ind_buf + M * NN;
         const PhysR<double> P64 = PhysR<double>::from(kc.phys);
-        const VinvRows<DIM, N> V = vinv_rows<DIM, N>(kc.Vinv, node);
+        const VinvRows<DIM, N> V = vinv_rows<DIM, N>(in_global(kc.Vinv), node);
         double m = 0.0;
         if (last && valid) m = Euler<DIM>::indicator_variable(uo, P64, kc.ind_var);
 #pragma unroll
