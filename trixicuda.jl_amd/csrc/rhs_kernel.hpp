@@ -131,7 +131,6 @@ template <typename R>
 using RhsConstArg = std::conditional_t<std::is_same<R, double>::value, const RhsConst* __restrict__, RhsConst>;
 __device__ __forceinline__ const RhsConst& consts_of(const RhsConst* p) { return *p; }
 __device__ __forceinline__ const RhsConst& consts_of(const RhsConst& v) { return v; }
-
 // A pointer read from the constants, known to point to global memory (as one that is
 // a kernel argument is): its loads are otherwise flat ones, which wait for LDS too.
 template <typename T>
@@ -302,6 +301,12 @@ rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
     constexpr bool LF = log_free<EQ, R, TW>();
     constexpr bool NODE_LOGS = !LF && (SF_LOGS || VF_LOGS || FV_LOGS);
     constexpr int NDF = NODE_LOGS ? 2 : 0;
+    // rhs!: the element's scale is read where it is used, except where reading it
+    // ahead of the fluxes was measured to gain (2D in FP64, and with FP32 arithmetic
+    // for fluxes with logarithms and the weak form on periodic meshes; 3D: weak form
+    // FP64 83.2 -> 81.5 us late, mixed 63.1 -> 62.3 at 32768 elements)
+    constexpr bool SCALE_LATE =
+        !RK && (DIM == 3 || (std::is_same<R, float>::value && VOL == VI_FD && (EXT || !VF_LOGS)));
     using Node = typename EQ::template Node<R, L>;
     // mixed precision weak form with N = 4 on whole waves: D-hat on MFMA
     constexpr bool WEAK_MFMA = TRIXI_HIP_WEAK_MFMA && VOL == VI_WEAK && std::is_same<R, float>::value &&
@@ -402,7 +407,7 @@ rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
 
     // the scale of the element's sums (a lane's nodes of the final pass belong to
     // its element too: NT is a multiple of M) and dt, ahead of the fluxes
-    const double invj = a.invJ[ec];
+    const double invj_early = SCALE_LATE ? 0.0 : a.invJ[ec];
     double t_dt = 0.0;
     if (RK) t_dt = a.time[1];
     double tnow = 0.0;
@@ -497,9 +502,8 @@ rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
 
     // last direction, sequential or not: -1/J (+ sources), then du or the RK update
     auto line_epilogue = [&](R (&al)[N][NV], int base, int s) {
-        const double fac = (TW ? -0.5 : -1.0) * invj;
-#pragma unroll
-        for (int p = 0; p < N; ++p) {
+        const double fac = (TW ? -0.5 : -1.0) * (SCALE_LATE ? a.invJ[e] : invj_early);
+        auto node_out = [&](int p, const R (&ap)[NV]) {
             const int node = base + p * s;
             double sv[NV];
 #pragma unroll
@@ -507,7 +511,7 @@ rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
             if (EXT && kc.src) source_at<DIM, NN, NV>(a, kc, e, node, tnow, sv);
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
-                R total = al[p][v];
+                R total = ap[v];
                 if (DIM > 1) total = acc[(v * NN + node) * LDM + el] + total;
                 const int64_t g = soa(v, node, e, slab, E32);
                 const double val = (double)total * fac + sv[v];
@@ -519,6 +523,25 @@ rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
                     UO[g] = (S)((double)U[g] + a.rk_b * (double)kk);
                 }
             }
+        };
+        if constexpr (EXT && DIM == 2 && NV <= 5 && std::is_same<R, float>::value) {
+            // one copy of the source terms' code instead of one per node, whose
+            // constants alone spilled (256 registers and 350 bytes of scratch a lane
+            // -> 132 and none; FP64 and 3D gain nothing from it)
+#pragma unroll 1
+            for (int p = 0; p < N; ++p) {
+                R ap[NV];
+#pragma unroll
+                for (int v = 0; v < NV; ++v) {
+                    ap[v] = al[0][v];
+#pragma unroll
+                    for (int q = 1; q < N; ++q) ap[v] = p == q ? al[q][v] : ap[v];
+                }
+                node_out(p, ap);
+            }
+        } else {
+#pragma unroll
+            for (int p = 0; p < N; ++p) node_out(p, al[p]);
         }
     };
 
@@ -858,7 +881,7 @@ rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
             const int n = q / M;
             const int64_t ee = e0 + c;
             if (ee >= E) continue;
-            const double fac = (TW ? -0.5 : -1.0) * invj;
+            const double fac = (TW ? -0.5 : -1.0) * invj_early;
             double sv[NV];
 #pragma unroll
             for (int v = 0; v < NV; ++v) sv[v] = 0.0;
