@@ -207,7 +207,8 @@ __device__ __forceinline__ R inv_ln_mean_logs(R x, R y, L lx, L ly) {
 // series below |z| = 0.01, the FP64 kernels drop the logarithms, their LDS and
 // registers, and every select and branch of a pair.
 // ---------------------------------------------------------------------------
-constexpr int MEANS_NEAR = 1, MEANS_ANY = 2;
+// MEANS_LOGS: from the nodes' logarithms after all.
+constexpr int MEANS_LOGS = 0, MEANS_NEAR = 1, MEANS_ANY = 2;
 
 // v_min_f64 / v_max_f64 as they are (fmin and fmax first quiet each operand
 // with an instruction of its own); a NaN operand yields the other one
@@ -1624,7 +1625,7 @@ __device__ __forceinline__ void node_flux(const typename EQ::template Node<R, L>
                                           const PhysR<R>& P, R* f) {
     if constexpr (TWICE)
         EQ::template twice_flux<KIND, MEANS>(l, ul, r, ur, o, P, f);
-    else if constexpr (log_free<EQ, R, TWICE>() && flux_needs_logs(KIND))
+    else if constexpr (MEANS != MEANS_LOGS && log_free<EQ, R, TWICE>() && flux_needs_logs(KIND))
         EQ::template two_point_log_free<KIND, MEANS>(l, r, o, P, f);
     else
         EQ::template two_point<KIND>(l, r, o, P, f);

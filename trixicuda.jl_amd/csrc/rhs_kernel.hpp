@@ -298,7 +298,12 @@ rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
     // FP64 Euler: fluxes and accumulators hold twice their value (TW); no node
     // logarithms there, nor in the FP64 MHD kernels (LF)
     constexpr bool TW = twice_fluxes<EQ, R, VOL, VF, SF, FVF>();
-    constexpr bool LF = log_free<EQ, R, TW>();
+    // (3D lines of five GLM-MHD nodes spill: their FP64 records carry logarithms,
+    // and no means are taken twice; rhs! at 4096 elements of shock capturing with
+    // the means' two paths 247 us and 768 bytes of scratch a lane, with logarithms
+    // 167 and 196)
+    constexpr bool LF = log_free<EQ, R, TW>() && !(EQ::NONCONS && DIM == 3 && N > 4);
+    constexpr int NEAR = LF ? MEANS_NEAR : MEANS_LOGS, ANY = LF ? MEANS_ANY : MEANS_LOGS;
     constexpr bool NODE_LOGS = !LF && (SF_LOGS || VF_LOGS || FV_LOGS);
     constexpr int NDF = NODE_LOGS ? 2 : 0;
     // rhs!: the element's scale is read where it is used, except where reading it
@@ -564,7 +569,7 @@ rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
 #pragma unroll 1
                 for (int j = i + 1; j < N; ++j) {
                     R f[NV];
-                    node_flux<EQ, VF, TW, MEANS_ANY, R, L>(staged_node(base + i * s), nullptr,
+                    node_flux<EQ, VF, TW, ANY, R, L>(staged_node(base + i * s), nullptr,
                                                            staged_node(base + j * s), nullptr, d, P, f);
                     const R fa = sc * (R)kc.Ds[i * N + j];
                     const R fb = sc * (R)kc.Ds[j * N + i];
@@ -698,7 +703,7 @@ rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
 #pragma unroll
                     for (int j = i + 1; j < N; ++j) {
                         R f[NV];
-                        node_flux<EQ, VF, TW, MEANS_NEAR, R, L>(nd[i], nullptr, nd[j], nullptr, d, P, f);
+                        node_flux<EQ, VF, TW, NEAR, R, L>(nd[i], nullptr, nd[j], nullptr, d, P, f);
                         const R fa = sc * (R)kc.Ds[i * N + j];
                         const R fb = sc * (R)kc.Ds[j * N + i];
 #pragma unroll
@@ -744,7 +749,7 @@ rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
                             ur[v] = nd[p + 1].cons(v);
                         }
                     }
-                    node_flux<EQ, FVF, TW, MEANS_ANY, R, L>(nd[p], ul, nd[p + 1], ur, d, P, F);
+                    node_flux<EQ, FVF, TW, ANY, R, L>(nd[p], ul, nd[p + 1], ur, d, P, F);
                     const R wl = alpha * (R)kc.invw[p];
                     const R wr = alpha * (R)kc.invw[p + 1];
                     if constexpr (EQ::NONCONS) {
@@ -782,8 +787,8 @@ rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
                     u1[v] = nd[N - 1].cons(v);
                 }
             }
-            node_flux<EQ, SF, TW, MEANS_ANY, R, L>(ndm, um, nd[0], u0, d, P, fm);      // this element is "right"
-            node_flux<EQ, SF, TW, MEANS_ANY, R, L>(nd[N - 1], u1, ndp, up, d, P, fp);  // this element is "left"
+            node_flux<EQ, SF, TW, ANY, R, L>(ndm, um, nd[0], u0, d, P, fm);      // this element is "right"
+            node_flux<EQ, SF, TW, ANY, R, L>(nd[N - 1], u1, ndp, up, d, P, fp);  // this element is "left"
             if constexpr (EQ::NONCONS) {
                 R ncm[NV], ncp[NV];
                 EQ::template noncons<SF>(nd[0], ndm, d, P, ncm);
