@@ -26,6 +26,10 @@ constexpr int group_elems() {
     while (m > 1 && m * 8 * (NRF * NN + NV * NN + DIM * 2 * NL * NV) > TRIXI_HIP_GROUP_LDS_KIB * 1024) m /= 2;
     return m;
 }
+// element lines from which lines_when_large forms take lines
+#ifndef TRIXI_HIP_GROUP_LINE_LANES
+#define TRIXI_HIP_GROUP_LINE_LANES 65536
+#endif
 #ifndef TRIXI_HIP_GROUP_WAVES2D
 #define TRIXI_HIP_GROUP_WAVES2D 3
 #endif
@@ -34,6 +38,21 @@ constexpr bool group_eligible() {
     return std::is_same<R, double>::value && DIM > 1 && VOL != VI_WEAK && HasRotation<EQ>::value &&
            (group_elems<DIM, N, EQ::NV, EQ::NRF>() * cpow(N, DIM - 1)) % 64 == 0 &&
            group_threads<DIM, N, group_elems<DIM, N, EQ::NV, EQ::NRF>()>() <= 1024;
+}
+
+// rhs! in 2D, and of Euler's shock capturing in 3D, takes the line form on meshes that
+// fill the GPU with it (a wave per SIMD and direction): its rows are as wide there,
+// and it has no group that the others wait for.  rhs! in us, lane groups / lines: 2D
+// at 16384 elements GLM-MHD 17.6 / 15.2, shock capturing 16.0 / 15.2; at 65536 Euler
+// 22.2 / 19.8, without logarithms 19.6 / 15.7, shock capturing 44.8 / 42.3; 3D Euler
+// shock capturing at 4096 32.9 / 31.5, at 32768 176 / 170.  Below, lane groups have
+// more lanes (2D GLM-MHD at 4096 8.3 / 12).  The RK stages, which read u and k
+// besides, gain from lane groups everywhere (2D GLM-MHD at 65536 94 / 156), and so do
+// 3D flux differencing (Euler at 32768 80 / 84) and 3D GLM-MHD (shock capturing at
+// 4096 53.5 / 55.0).
+template <int DIM, class EQ, int VOL, bool RK, bool EXT>
+constexpr bool lines_when_large() {
+    return !RK && !EXT && (DIM == 2 || (VOL == VI_HG && !EQ::NONCONS));
 }
 
 // Launch helper used by the instantiation units: the node-parallel form for
@@ -69,13 +88,20 @@ hipError_t launch_rhs(const RhsArgs& a, hipStream_t stream) {
         // waves spill: boundary and mortar faces, and shock capturing in 3D,
         // whose blended lines hold 60 registers too many (rhs! at 32768
         // elements 219 -> 180 us, three CFL steps 4360 -> 3320; with three
-        // waves the same).
-        constexpr bool HALF = EXT || (VOL == VI_HG && DIM == 3);
+        // waves the same).  In 2D the tiles cannot be halved (whole waves), and
+        // three waves hold boundary and mortar faces as well (65536 elements with
+        // Dirichlet faces: rhs! 48.3 -> 37.0 us, RK stage 63.9 -> 51.4).
+        constexpr bool HALF = (EXT || VOL == VI_HG) && DIM == 3;
         constexpr int MG = HALF && (ME / 2 * cpow(N, DIM - 1)) % 64 == 0 ? ME / 2 : ME;
         constexpr int W = EQ::NV > 5 || HALF ? 2 : (DIM == 3 ? 4 : TRIXI_HIP_GROUP_WAVES2D);
-        hipLaunchKernelGGL((rhs_group_kernel<DIM, N, EQ, VOL, VF, SF, FVF, MG, RK, EXT, W>), grid(MG),
-                           dim3(group_threads<DIM, N, MG>()), 0, stream, a, a.consts);
-    } else {
+        constexpr bool LINES = lines_when_large<DIM, EQ, VOL, RK, EXT>();
+        if (!LINES || a.E * cpow(N, DIM - 1) < TRIXI_HIP_GROUP_LINE_LANES) {
+            hipLaunchKernelGGL((rhs_group_kernel<DIM, N, EQ, VOL, VF, SF, FVF, MG, RK, EXT, W>), grid(MG),
+                               dim3(group_threads<DIM, N, MG>()), 0, stream, a, a.consts);
+            return hipGetLastError();
+        }
+    }
+    if constexpr (!group_eligible<DIM, N, EQ, VOL, R>() || lines_when_large<DIM, EQ, VOL, RK, EXT>()) {
         hipLaunchKernelGGL((rhs_kernel<DIM, N, EQ, VOL, VF, SF, FVF, R, M, RK, EXT, L, S>), grid(M),
                            dim3(rhs_threads<DIM, N, M, R, RK, EQ::NV>()), 0, stream, a, consts());
     }
