@@ -715,6 +715,16 @@ using namespace trixi_hip;
 // ---------------------------------------------------------------------------
 // context
 // ---------------------------------------------------------------------------
+// The small device data of a context, one allocation and one copy (seven and six of
+// their own were a sixth of the set-up of a 4096-element context).  What kernels write
+// lies in cache lines of its own.
+struct CtxSmall {
+    RhsConst consts;
+    double Vinv[MAXN * MAXN], Vdm[(2 * MAXN - 1) * MAXN], wa[2 * MAXN - 1], w[MAXN];
+    alignas(128) double time[TIME_DOUBLES];
+    alignas(128) unsigned arrived[ARRIVAL_COUNTERS];
+};
+
 struct trixi_hip_ctx {
     trixi_hip_config cfg;
     int dim, N, nv, nn;
@@ -729,19 +739,20 @@ struct trixi_hip_ctx {
     double* d_x = nullptr;
     double* d_alpha_raw = nullptr;
     double* d_alpha = nullptr;
-    double* d_time = nullptr;
+    CtxSmall* d_small = nullptr;   // holds the members marked (s)
+    double* d_time = nullptr;      // (s)
     double* d_partial = nullptr;
     double* h_result = nullptr;    // pinned: the last block of a reduction writes here
-    unsigned* d_arrived = nullptr;  // blocks of a running reduction that have arrived [ARRIVAL_COUNTERS]
-    double* d_Vinv = nullptr;
-    double* d_Vdm = nullptr;
-    double* d_wa = nullptr;
-    double* d_w = nullptr;
+    unsigned* d_arrived = nullptr;  // (s) blocks of a running reduction that have arrived [ARRIVAL_COUNTERS]
+    double* d_Vinv = nullptr;       // (s)
+    double* d_Vdm = nullptr;        // (s)
+    double* d_wa = nullptr;         // (s)
+    double* d_w = nullptr;          // (s)
     double* d_tmp = nullptr;  // RK stage states (two buffers of nvalues)
     int nblocks_red = 1024;
     RhsArgs args;
     RhsConst consts;               // as on the device
-    RhsConst* d_consts = nullptr;
+    RhsConst* d_consts = nullptr;  // (s)
     LaunchFn rhs_fn = nullptr, rk_fn = nullptr;
     // adjoint
     VjpFn vjp_fn = nullptr;
@@ -814,8 +825,7 @@ static void free_ctx(trixi_hip_ctx* c) {
     if (!c) return;
     if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
     if (c->graph) (void)hipGraphDestroy(c->graph);
-    void* bufs[] = {c->d_nbr, c->d_invJ, c->d_x,     c->d_alpha_raw, c->d_alpha, c->d_time,
-                    c->d_partial, c->d_arrived, c->d_consts, c->d_Vinv, c->d_Vdm,   c->d_wa,    c->d_w,
+    void* bufs[] = {c->d_nbr, c->d_invJ, c->d_x, c->d_alpha_raw, c->d_alpha, c->d_small, c->d_partial,
                     c->d_tmp, c->d_stage, c->d_k, c->d_kbar, c->d_alphabar, c->d_winner, c->d_stage_alpha,
                     c->d_mids, c->d_mori, c->d_mls, c->d_mnb, c->d_mflux};
     for (void* p : bufs)
@@ -1165,19 +1175,18 @@ int trixi_hip_create(const trixi_hip_config* config, const trixi_hip_mesh* mesh,
     ALLOC(c->d_x, (size_t)dim * nn * E * sizeof(double));
     ALLOC(c->d_alpha_raw, E * sizeof(double));
     ALLOC(c->d_alpha, E * sizeof(double));
-    ALLOC(c->d_time, TIME_DOUBLES * sizeof(double));
+    ALLOC(c->d_small, sizeof(CtxSmall));
+    c->d_time = c->d_small->time;
+    c->d_arrived = c->d_small->arrived;
+    c->d_consts = &c->d_small->consts;
+    c->d_Vinv = c->d_small->Vinv;
+    c->d_Vdm = c->d_small->Vdm;
+    c->d_wa = c->d_small->wa;
+    c->d_w = c->d_small->w;
     ALLOC(c->d_partial, (size_t)c->nblocks_red * 18 * sizeof(double));
-    ALLOC(c->d_arrived, ARRIVAL_COUNTERS * sizeof(unsigned));
-    ALLOC(c->d_consts, sizeof(RhsConst));
     c->h_result = take_result_slot();
     if (!c->h_result)
         return cleanup_fail(TRIXI_HIP_ENOMEM, "hipHostMalloc failed for the reduction results");
-    if (hipMemset(c->d_arrived, 0, ARRIVAL_COUNTERS * sizeof(unsigned)) != hipSuccess)
-        return cleanup_fail(TRIXI_HIP_EDEVICE, "hipMemset failed in create");
-    ALLOC(c->d_Vinv, N * N * sizeof(double));
-    ALLOC(c->d_Vdm, c->NA * N * sizeof(double));
-    ALLOC(c->d_wa, c->NA * sizeof(double));
-    ALLOC(c->d_w, N * sizeof(double));
     ALLOC(c->d_tmp, 2 * (size_t)c->nvalues * sizeof(double));
     if (NM > 0) {
         const size_t slots = (size_t)NM * (K + 1);
@@ -1203,15 +1212,17 @@ int trixi_hip_create(const trixi_hip_config* config, const trixi_hip_mesh* mesh,
     } else {
         ok = ok && hipMemset(c->d_x, 0, (size_t)dim * nn * E * sizeof(double)) == hipSuccess;
     }
-    ok = ok && up(c->d_Vinv, c->basis.Vinv.data(), N * N * sizeof(double));
+    CtxSmall small;
+    memset(&small, 0, sizeof small);
     {
         std::vector<double> xa, wa;
         lgl(c->NA, xa, wa);
-        std::vector<double> V = interpolation_matrix(c->basis.x, c->basis.wbary, xa);
-        ok = ok && up(c->d_Vdm, V.data(), V.size() * sizeof(double));
-        ok = ok && up(c->d_wa, wa.data(), wa.size() * sizeof(double));
+        const std::vector<double> V = interpolation_matrix(c->basis.x, c->basis.wbary, xa);
+        std::copy(c->basis.Vinv.begin(), c->basis.Vinv.end(), small.Vinv);
+        std::copy(V.begin(), V.end(), small.Vdm);
+        std::copy(wa.begin(), wa.end(), small.wa);
+        std::copy(c->basis.w.begin(), c->basis.w.end(), small.w);
     }
-    ok = ok && up(c->d_w, c->basis.w.data(), N * sizeof(double));
     if (NM > 0) {
         ok = ok && up(c->d_mids, mesh->mortar_neighbor_ids, (size_t)NM * (K + 1) * sizeof(int32_t));
         ok = ok && up(c->d_mori, mesh->mortar_orientations, NM * sizeof(int32_t));
@@ -1322,7 +1333,8 @@ int trixi_hip_create(const trixi_hip_config* config, const trixi_hip_mesh* mesh,
                       !(fenv && atoi(fenv) == 0);
     }
     {
-        if (hipMemcpy(c->d_consts, &c->consts, sizeof(RhsConst), hipMemcpyHostToDevice) != hipSuccess)
+        small.consts = c->consts;
+        if (!up(c->d_small, &small, sizeof small))
             return cleanup_fail(TRIXI_HIP_EDEVICE, "host to device copy failed in create");
         // look up this device's static scratch once, at set-up, with the
         // device current (used by the *_noalloc entry points)
