@@ -309,9 +309,10 @@ rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
     // rhs!: the element's scale is read where it is used, except where reading it
     // ahead of the fluxes was measured to gain (2D in FP64, and with FP32 arithmetic
     // for fluxes with logarithms and the weak form on periodic meshes; 3D: weak form
-    // FP64 83.2 -> 81.5 us late, mixed 63.1 -> 62.3 at 32768 elements)
-    constexpr bool SCALE_LATE =
-        !RK && (DIM == 3 || (std::is_same<R, float>::value && VOL == VI_FD && (EXT || !VF_LOGS)));
+    // FP64 83.2 -> 81.5 us late, mixed 63.1 -> 62.3 at 32768 elements, but with
+    // mortars linear advection at 36352 elements 72.1 -> 73.9)
+    constexpr bool SCALE_LATE = !RK && ((DIM == 3 && !EXT) || (std::is_same<R, float>::value && DIM == 2 &&
+                                                              VOL == VI_FD && (EXT || !VF_LOGS)));
     using Node = typename EQ::template Node<R, L>;
     // mixed precision weak form with N = 4 on whole waves: D-hat on MFMA
     constexpr bool WEAK_MFMA = TRIXI_HIP_WEAK_MFMA && VOL == VI_WEAK && std::is_same<R, float>::value &&
@@ -529,10 +530,12 @@ rhs_kernel(const RhsArgs a, const RhsConstArg<R> consts) {
                 }
             }
         };
-        if constexpr (EXT && DIM == 2 && NV <= 5 && std::is_same<R, float>::value) {
+        if constexpr (EXT && DIM == 2 && IsEuler<EQ>::value && std::is_same<R, float>::value) {
             // one copy of the source terms' code instead of one per node, whose
-            // constants alone spilled (256 registers and 350 bytes of scratch a lane
-            // -> 132 and none; FP64 and 3D gain nothing from it)
+            // constants alone spilled (2D Euler with FP32 arithmetic: 256 registers and
+            // 350 bytes of scratch a lane -> 132 and none; with FP64 and in 3D the
+            // spills stay, and without source terms the loop costs: linear advection at
+            // 77824 elements 12.2 -> 12.8 us)
 #pragma unroll 1
             for (int p = 0; p < N; ++p) {
                 R ap[NV];
