@@ -608,19 +608,21 @@ struct Euler {
         }
     }
     // whether every pair of these nodes satisfies MEANS_NEAR: rho, and rho / p
-    // through the staged sound speed (rho / p = gamma / c^2)
+    // through the staged sound speed (rho / p = gamma / c^2).  Minimum and maximum
+    // pass over a node that is not a number; the sum of the speeds does not, nor one
+    // with p / rho < 0
     template <int N, class ND>
     __device__ static bool near_line(const ND* n) {
-        double r0 = n[0].rho, r1 = r0, c0 = n[0].c, c1 = c0, p0 = n[0].p;
+        double r0 = n[0].rho, r1 = r0, c0 = n[0].c, c1 = c0, sum = c0;
 #pragma unroll
         for (int i = 1; i < N; ++i) {
             r0 = raw_min(r0, n[i].rho);
             r1 = raw_max(r1, n[i].rho);
             c0 = raw_min(c0, n[i].c);
             c1 = raw_max(c1, n[i].c);
-            p0 = raw_min(p0, n[i].p);
+            sum += n[i].c;
         }
-        const bool a = near_ratio(r0, r1), b = near_ratio(c0 * c0, c1 * c1), c = p0 > 0.0;
+        const bool a = near_ratio(r0, r1), b = near_ratio(c0 * c0, c1 * c1), c = sum < 0x1p1000;
         return a && b && c && near_range(n[0].rho, n[0].p);
     }
 
@@ -1432,10 +1434,11 @@ struct GlmMhd {
         }
     }
     // whether every pair of these nodes satisfies MEANS_NEAR: rho, and rho / p
-    // (v_rcp_f64 as it is: within 2^-24, far inside the polynomials' margin)
+    // (v_rcp_f64 as it is: within 2^-24, far inside the polynomials' margin); false
+    // for a node that is not a number
     template <int N, typename L>
     __device__ static bool near_line(const Node<double, L>* n) {
-        double r0 = n[0].rho, r1 = r0, b0 = r0 * __builtin_amdgcn_rcp(n[0].p), b1 = b0;
+        double r0 = n[0].rho, r1 = r0, b0 = r0 * __builtin_amdgcn_rcp(n[0].p), b1 = b0, sum = n[0].p;
 #pragma unroll
         for (int i = 1; i < N; ++i) {
             const double b = n[i].rho * __builtin_amdgcn_rcp(n[i].p);
@@ -1443,8 +1446,9 @@ struct GlmMhd {
             r1 = raw_max(r1, n[i].rho);
             b0 = raw_min(b0, b);
             b1 = raw_max(b1, b);
+            sum += n[i].p;
         }
-        const bool a = near_ratio(r0, r1), b = near_ratio(b0, b1);
+        const bool a = near_ratio(r0, r1), b = near_ratio(b0, b1) && sum < 0x1p1000;
         return a && b && near_range(n[0].rho, n[0].p);
     }
 
