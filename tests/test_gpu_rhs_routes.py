@@ -21,7 +21,8 @@ LARGE = (
     + [Case(f"mhd2d_hg_{s}", 2, "mhd", 7, "hg", HG, s, s, gamma=5 / 3, alpha_min=0.0) for s in ("llf", HG)]
     + [Case(f"euler3d_hg_{v}_{s}", 3, "euler", 4, "hg", v, s, s, alpha_min=0.0)
        for v, s in (("ranocha", "llf"), ("ranocha", "llf_naive"), ("ranocha", "ranocha"), ("shima_etal", "llf"),
-                    ("shima_etal", "llf_naive"))])
+                    ("shima_etal", "llf_naive"))]
+    + [Case("euler3d_hg_level5", 3, "euler", 5, "hg", "ranocha", alpha_min=0.0)])
 
 
 @pytest.mark.parametrize("case", LARGE, ids=lambda c: c.name)
