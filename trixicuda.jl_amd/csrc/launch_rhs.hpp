@@ -40,24 +40,20 @@ constexpr bool group_eligible() {
            group_threads<DIM, N, group_elems<DIM, N, EQ::NV, EQ::NRF>()>() <= 1024;
 }
 
-// rhs! in 2D, and of Euler's shock capturing in 3D, takes the line form on meshes that
-// fill the GPU with it (a wave per SIMD and direction): its rows are as wide there,
-// and it has no group that the others wait for.  rhs! in us, lane groups / lines: 2D
-// at 16384 elements GLM-MHD 17.6 / 15.2, shock capturing 16.0 / 15.2; at 65536 Euler
-// 22.2 / 19.8, without logarithms 19.6 / 15.7, shock capturing 44.8 / 42.3; 3D Euler
-// shock capturing at 4096 33.0 / 33.8, without logarithms 32.9 / 31.5, at 32768 176 /
-// 170 and 174 / 166.  Below, lane groups have more lanes (2D GLM-MHD at 4096 8.3 / 12).  The RK stages, which read u and k
-// besides, gain from lane groups everywhere (2D GLM-MHD at 65536 94 / 156), and so do
-// 3D flux differencing (Euler at 32768 80 / 84) and 3D GLM-MHD (shock capturing at
-// 4096 53.5 / 55.0).
-template <int DIM, class EQ, int VOL, bool RK, bool EXT>
+// rhs! in 2D, and of Euler's shock capturing without logarithmic means in 3D, takes
+// the line form on meshes that fill the GPU with it (a wave per SIMD and direction):
+// its rows are as wide there, and it has no group that the others wait for.  rhs! in
+// us, lane groups / lines: 2D at 16384 elements GLM-MHD 17.6 / 15.2, shock capturing
+// 16.0 / 15.2; at 65536 Euler 21.0 / 18.8, without logarithms 19.6 / 15.7, shock
+// capturing 44.8 / 42.8; 3D shock capturing without logarithms at 4096 32.9 / 31.4, at
+// 32768 173 / 165.  Below, lane groups have more lanes (2D GLM-MHD at 4096 8.3 / 12).
+// The RK stages, which read u and k besides, gain from lane groups everywhere (2D
+// GLM-MHD at 65536 94 / 156), and so do 3D flux differencing (Euler at 32768 80 / 84),
+// 3D shock capturing with logarithms (at 4096 33.0 / 33.8, at 32768 176 / 187) and 3D
+// GLM-MHD (shock capturing at 4096 53.5 / 55.0).
+template <int DIM, class EQ, int VOL, int VF, bool RK, bool EXT>
 constexpr bool lines_when_large() {
-    return !RK && !EXT && (DIM == 2 || (VOL == VI_HG && !EQ::NONCONS));
-}
-// element lines of a large mesh
-template <int DIM, int VF>
-constexpr int64_t large_lanes() {
-    return (DIM == 3 && flux_needs_logs(VF) ? 4 : 1) * (int64_t)TRIXI_HIP_GROUP_LINE_LANES;
+    return !RK && !EXT && (DIM == 2 || (VOL == VI_HG && !EQ::NONCONS && !flux_needs_logs(VF)));
 }
 
 // Launch helper used by the instantiation units: the node-parallel form for
@@ -99,14 +95,14 @@ hipError_t launch_rhs(const RhsArgs& a, hipStream_t stream) {
         constexpr bool HALF = (EXT || VOL == VI_HG) && DIM == 3;
         constexpr int MG = HALF && (ME / 2 * cpow(N, DIM - 1)) % 64 == 0 ? ME / 2 : ME;
         constexpr int W = EQ::NV > 5 || HALF ? 2 : (DIM == 3 ? 4 : TRIXI_HIP_GROUP_WAVES2D);
-        constexpr bool LINES = lines_when_large<DIM, EQ, VOL, RK, EXT>();
-        if (!LINES || a.E * cpow(N, DIM - 1) < large_lanes<DIM, VF>()) {
+        constexpr bool LINES = lines_when_large<DIM, EQ, VOL, VF, RK, EXT>();
+        if (!LINES || a.E * cpow(N, DIM - 1) < TRIXI_HIP_GROUP_LINE_LANES) {
             hipLaunchKernelGGL((rhs_group_kernel<DIM, N, EQ, VOL, VF, SF, FVF, MG, RK, EXT, W>), grid(MG),
                                dim3(group_threads<DIM, N, MG>()), 0, stream, a, a.consts);
             return hipGetLastError();
         }
     }
-    if constexpr (!group_eligible<DIM, N, EQ, VOL, R>() || lines_when_large<DIM, EQ, VOL, RK, EXT>()) {
+    if constexpr (!group_eligible<DIM, N, EQ, VOL, R>() || lines_when_large<DIM, EQ, VOL, VF, RK, EXT>()) {
         hipLaunchKernelGGL((rhs_kernel<DIM, N, EQ, VOL, VF, SF, FVF, R, M, RK, EXT, L, S>), grid(M),
                            dim3(rhs_threads<DIM, N, M, R, RK, EQ::NV>()), 0, stream, a, consts());
     }
