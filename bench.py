@@ -336,9 +336,10 @@ def main():
             "value": dofs / secs, "ms_per_step": ms, "wall_ms_per_step": wall_ms,
             "roofline": {"bound": "hbm", "achieved": gbps, "peak": fm.PEAK["hbm_GBps"], "unit": "GB/s",
                          "frac": gbps / fm.PEAK["hbm_GBps"], "traffic": traffic.get(mode),
-                         "kernel": "rhs_kernel<3, 4, Euler<3>, FD, flux_ranocha, LLF, "
-                                   + {"fp64": "double, M=4>", "mixed": "float, M=16, logs double>",
-                                      "fp32": "float, M=16, logs float, state float>"}[mode],
+                         "kernel": {"fp64": "rhs_group_kernel<3, 4, Euler<3>, FD, flux_ranocha, LLF, M=8>",
+                                    "mixed": "rhs_kernel<3, 4, Euler<3>, FD, flux_ranocha, LLF, float, M=16, logs double>",
+                                    "fp32": "rhs_kernel<3, 4, Euler<3>, FD, flux_ranocha, LLF, float, M=16, logs float, "
+                                            "state float>"}[mode],
                          "algorithmic_bytes": bytes_dof * dofs, "bytes_per_dof": bytes_dof,
                          "flop_per_dof": flops_dof, "flop_TFLOPs": achieved_tf, "flop_peak_TFLOPs": fpeak,
                          "flop_frac": achieved_tf / fpeak},

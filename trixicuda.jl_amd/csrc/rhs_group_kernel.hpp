@@ -23,7 +23,7 @@
 // Euler at 32768 elements 1985 -> 1720 us, five steps on a refined mesh of 960
 // elements 807 -> 647 us, rhs! alone at 32768 elements 83.7 -> 81.0 us (with
 // the device time loop, the constants behind a pointer and the loads ahead of
-// the fluxes now 1550, 568 and 79.9 us).  An XOR exchange of the node places
+// the fluxes now 1530, 561 and 78.9 us).  An XOR exchange of the node places
 // against the bank conflicts of x-lines (node_place in vjp_group_kernel.hpp)
 // gained 1 % for MHD and cost 1 % here and 3 % in 2D.  A
 // register spilled in this kernel costs more than everything else (each lane's

@@ -252,7 +252,8 @@ __device__ __forceinline__ int line_base(int line, int d) {
 // sequential form: FP64 rhs! and RK stages.  (Measured with 3D Euler flux
 // differencing at level 5, 93.8 -> 89.5 us, before that configuration had
 // rhs_group_kernel; what runs this form now are the FP64 weak forms, the
-// equations without a lane-group form and node counts that do not fill waves.)
+// equations without a lane-group form, node counts that do not fill waves, and
+// rhs! on large meshes where launch_rhs.hpp takes lines.)
 // In FP32 arithmetic (63.4 -> 76.8 us) the sequential form stays, with one
 // copy of each direction's code live at a time, and so it does for systems of
 // more than five variables, whose parallel form spills (3D GLM-MHD at level 4:

@@ -9,9 +9,9 @@
 // from LDS, so that four waves per SIMD fit (128 registers); node_place keeps
 // those reads free of bank conflicts, log_free_mean_grads needs no logarithms,
 // and the volume code has its direction as a constant, so that field offsets are
-// part of the load instructions.  What is left is FP64 issue (60 % of the time;
-// 34 million wave instructions at 32768 elements) and the waits of a workgroup's
-// first pass and barriers.
+// part of the load instructions.  What is left is FP64 issue (34 million wave
+// instructions at 32768 elements, half of the VALU's slots at 105 us on one pair of
+// buffers) and the waits of a workgroup's first pass and barriers.
 //
 // 3D Euler at 32768 elements 168 -> 124 us (136 with the direction as data, 130
 // before the fluxes' adjoints were shortened; tiles of 4 elements 143); 2D Euler
